@@ -1,4 +1,5 @@
-"""ctypes binding of libmambaqc_hip.so (declared in include/mambaqc_hip.h).
+"""ctypes binding of libmambaqc_hip.so (declared in include/mambaqc_hip.h
+and include/mambaqc_hip_ext.h).
 
 The library is the only compute path of this package: there is no CPU or
 torch fallback. Loading fails loudly with the build command if the library is
@@ -85,6 +86,15 @@ SIGNATURES_I64 = {
     "mqc_ssm_fused_bc_split_workspace_bytes": [_i64, _i64, _i64, _i64],
 }
 
+# The same for the entry points of include/mambaqc_hip_ext.h.
+SIGNATURES_EXT = {
+    "mqc_gemm_f32": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64,
+                     _vp],
+}
+SIGNATURES_EXT_I64 = {
+    "mqc_gemm_f32_workspace_bytes": [_i64, _i64, _i64],
+}
+
 ABI_VERSION = 8
 
 _lock = threading.Lock()
@@ -109,11 +119,11 @@ def load(path: os.PathLike | str | None = None) -> ctypes.CDLL:
                 f"{p} is missing: build it with `python -m mambaqc_amd.build` "
                 "(mambaqc_amd has no CPU fallback)")
         lib = ctypes.CDLL(str(p))
-        for name, argtypes in SIGNATURES.items():
+        for name, argtypes in {**SIGNATURES, **SIGNATURES_EXT}.items():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = _int
-        for name, argtypes in SIGNATURES_I64.items():
+        for name, argtypes in {**SIGNATURES_I64, **SIGNATURES_EXT_I64}.items():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = _i64

@@ -10,7 +10,7 @@
 
 #include <type_traits>
 
-#include "../../include/mambaqc_hip.h"
+#include "../../include/mambaqc_hip_ext.h"
 
 namespace mqc {
 

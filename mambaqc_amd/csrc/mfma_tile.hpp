@@ -169,7 +169,12 @@ __device__ inline void tile_issue_stage(int kt, int wave, uint32_t lds0, const D
   }
 }
 
-template <typename Cfg, typename E = __bf16, typename WRow, typename XRow>
+//
+// SPLIT: each row holds an fp32 row as two fp16 pieces (gemm_f32.hip), a K step's 128 bytes
+// being 32 columns' high pieces and then the same columns' low pieces, so the two "K slices"
+// of a step are W_hi, W_lo and X_hi, X_lo, and the step's products are W_hi X_hi, W_hi X_lo
+// and W_lo X_hi: half as many MFMAs again per byte staged.
+template <typename Cfg, typename E = __bf16, bool SPLIT = false, typename WRow, typename XRow>
 __device__ inline void tile_kloop_cfg(int K, char* lds,
                                       floatx4 (&acc)[Cfg::WB][Cfg::XB], const WRow& wrow,
                                       const XRow& xrow) {
@@ -204,12 +209,12 @@ __device__ inline void tile_kloop_cfg(int K, char* lds,
 #pragma unroll
     for (int mb = 0; mb < XB; ++mb) xf[buf][mb] = *(const frag*)(sb + xoff[kk] + mb * 16 * kRowBytes);
   };
-  auto mfmas = [&](int buf) {
+  auto mfmas = [&](int wbuf, int xbuf) {
 #pragma unroll
     for (int nb = 0; nb < WB; ++nb)
 #pragma unroll
       for (int mb = 0; mb < XB; ++mb)
-        acc[nb][mb] = mfma16(wf[buf][nb], xf[buf][mb], acc[nb][mb]);
+        acc[nb][mb] = mfma16(wf[wbuf][nb], xf[xbuf][mb], acc[nb][mb]);
   };
 
   const int KT = K / kBK;
@@ -224,14 +229,19 @@ __device__ inline void tile_kloop_cfg(int K, char* lds,
     __builtin_amdgcn_sched_barrier(0);
     // First K slice: its MFMAs with the second slice's fragment reads, one after each MFMA.
     read_frags(1, sbase, 1);
-    mfmas(0);
+    mfmas(0, 0);
 #pragma unroll
     for (int g = 0; g < WB + XB; ++g) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
     }
     __builtin_amdgcn_sched_barrier(0);
-    mfmas(1);
+    if constexpr (SPLIT) {
+      mfmas(0, 1);
+      mfmas(1, 0);
+    } else {
+      mfmas(1, 1);
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
 }

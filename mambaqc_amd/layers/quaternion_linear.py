@@ -134,6 +134,89 @@ class _WideLinearFunction(torch.autograd.Function):
         return dx, dw, None
 
 
+# fp32 products run on the library's split-fp16 GEMM (mqc_gemm_f32: fp32 accuracy on the
+# 16-bit matrix cores) where it is the faster one. Against hipBLASLt's fp32, which reaches
+# 115-153 of the fp32 matrix cores' 157 TFLOP/s, it multiplies at 300-380 TFLOP/s but first
+# splits both operands (8 bytes moved per element), so the shorter side of the product has to
+# repay that, and the whole one its extra launches. Measured on MI355X (us, library / this
+# GEMM): forward M 1024 N 131072 K 1024 1935 / 954, M 400 N 32768 K 512 129 / 75; input
+# gradients of the same 2223 / 1329 and 358 / 135; weight gradients 1912 / 1132 and 110 / 87.
+# Below the line: M 100 N 98304 K 384 86 / 120 (a short side), 98304 x 384 over K 100
+# 94 / 114 (short k: padding and output dominate), 1024 x 1024 x 1024 22 / 35 (launches).
+F32_GEMM_MIN_SIDE = 200     # M N / (M + N)
+F32_GEMM_MIN_K = 192
+F32_GEMM_MIN_FLOP = 6e9
+
+
+def _f32_gemm_shape(M: int, N: int, K: int) -> bool:
+    return (K >= F32_GEMM_MIN_K and M * N >= F32_GEMM_MIN_SIDE * (M + N)
+            and 2.0 * M * N * K >= F32_GEMM_MIN_FLOP)
+
+
+def _unit_rows(t: torch.Tensor) -> torch.Tensor:
+    """t [R, C] with one axis dense and no overlapping rows, copied only if it is not."""
+    ok = any(t.stride(i) == 1 and t.stride(1 - i) >= t.shape[i] for i in (0, 1))
+    return t if ok else t.contiguous()
+
+
+def _f32_mm_t(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T in fp32, x [M, K] and w [N, K] (or transposed views): on mqc_gemm_f32 where it
+    is faster, else torch's."""
+    M, K = x.shape
+    N = w.shape[0]
+    if not _f32_gemm_shape(M, N, K):
+        return torch.mm(x, w.t())
+    x, w = _unit_rows(x), _unit_rows(w)
+    lib = nat.load()
+    nbytes = int(lib.mqc_gemm_f32_workspace_bytes(M, N, K))
+    if nbytes < 0:
+        nat.check(nbytes, "mqc_gemm_f32_workspace_bytes")
+    y = torch.empty(M, N, device=x.device, dtype=torch.float32)
+    ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
+    nat.call("mqc_gemm_f32", x, x.data_ptr(), x.stride(0), x.stride(1), w.data_ptr(),
+             w.stride(0), w.stride(1), y.data_ptr(), N, M, N, K, ws.data_ptr(), nbytes,
+             nat.stream_of(x))
+    return y
+
+
+class _F32MatmulT(torch.autograd.Function):
+    """x w^T in fp32. Its gradients are products of the same kind (gy w and gy^T x), made by
+    the same function, so gradients of gradients exist as for torch's."""
+
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        return _f32_mm_t(x, w)
+
+    @staticmethod
+    def backward(ctx, gy):
+        x, w = ctx.saved_tensors
+        gx = _F32MatmulT.apply(gy, w.t()) if ctx.needs_input_grad[0] else None
+        gw = _F32MatmulT.apply(gy.t(), x.t()) if ctx.needs_input_grad[1] else None
+        return gx, gw
+
+
+def _plain_call(*tensors) -> bool:
+    """Plain dense tensors called eagerly: no tensor subclass (fake tensors), no dispatch
+    mode, tracing, functorch transform or forward-mode AD in progress, all of which torch's
+    own operators take part in and a direct launch does not."""
+    return (all(type(t) in (torch.Tensor, nn.Parameter) and t.layout == torch.strided and not t.is_neg()
+                for t in tensors)
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0)
+
+
+def _f32_linear_eligible(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    n, k = weight.shape
+    rows = x.numel() // k if k else 0
+    return (x.dtype == torch.float32 and weight.dtype == torch.float32
+            and x.is_cuda and weight.device == x.device and x.shape[-1] == k
+            and _f32_gemm_shape(rows, n, k) and _plain_call(x, weight)
+            and not torch.is_autocast_enabled(x.device.type))
+
+
 def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """F.linear(x, weight) without bias, computed as column blocks of the
     output whose weight rows fit WIDE_LINEAR_CHUNK_BYTES, each written in place
@@ -143,8 +226,13 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     Used on a GPU when the weight exceeds the bound and x has at least
     WIDE_LINEAR_MIN_ROWS rows; everything else takes F.linear. Under autocast
     the operands are cast to the autocast dtype, as F.linear's autocast rule
-    does. Each output element is the same K-reduction as in one launch.
+    does. Each output element is the same K-reduction as in one launch. fp32 products
+    that _f32_gemm_shape accepts run on the library's split GEMM instead, whatever their
+    weight's size.
     """
+    if _f32_linear_eligible(x, weight):
+        out = _F32MatmulT.apply(x.reshape(-1, x.shape[-1]), weight)
+        return out.view(*x.shape[:-1], weight.shape[0])
     n, k = weight.shape
     rows = x.numel() // k if k else 0
     if (n * k * weight.element_size() <= WIDE_LINEAR_CHUNK_BYTES or rows < WIDE_LINEAR_MIN_ROWS
