@@ -25,6 +25,20 @@ int mqc_gemm_f32(const float* X, int64_t x_row, int64_t x_col, const float* W, i
                  int64_t w_col, float* Y, int64_t ldy, int64_t M, int64_t N, int64_t K,
                  void* workspace, int64_t workspace_bytes, void* stream);
 
+/* mqc_ssm_fused_bc_fwd for short sequences, seq_len from 1 to 128 (MQC_E_LIMIT above): same
+ * operands, dtypes, shapes and refusals, in tiles of 64 or 128 tokens that hold whole
+ * sequences of the batch, each group of 16 states in a workgroup of its own. d_state > 16
+ * needs workspace (mqc_ssm_fused_bc_short_workspace_bytes, 16-byte aligned) for the groups'
+ * partial sums of y. h_last may be h0. */
+int64_t mqc_ssm_fused_bc_short_workspace_bytes(int64_t batch, int64_t seq_len, int64_t d_inner,
+                                               int64_t d_state);
+int mqc_ssm_fused_bc_short_fwd(const void* x, const void* B_weight, const void* C_weight,
+                               const void* delta, const void* s, const float* lambda_alpha,
+                               const float* lambda_imag, const float* D, const void* h0, void* y,
+                               void* h_last, int64_t batch, int64_t seq_len, int64_t d_inner,
+                               int64_t d_state, float eps, int dtype, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -90,8 +90,11 @@ SIGNATURES_I64 = {
 SIGNATURES_EXT = {
     "mqc_gemm_f32": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64,
                      _vp],
+    "mqc_ssm_fused_bc_short_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                   _i64, _i64, _i64, _i64, _f32, _int, _vp, _i64, _vp],
 }
 SIGNATURES_EXT_I64 = {
+    "mqc_ssm_fused_bc_short_workspace_bytes": [_i64, _i64, _i64, _i64],
     "mqc_gemm_f32_workspace_bytes": [_i64, _i64, _i64],
 }
 

@@ -43,13 +43,10 @@
 // the caller's workspace, and fused_bc_combine_kernel adds the halves and D s.
 #include <atomic>
 
-#include "mfma_tile.hpp"
-#include "ssm_chunk.hpp"
+#include "fused_bc.hpp"
 
 namespace mqc {
 namespace {
-
-using namespace mfma;
 
 constexpr int kHalf = 32;                 // states per half
 constexpr int kMaxHalves = 2;             // d_state <= 64
@@ -72,6 +69,8 @@ constexpr int kLdsFused = kOffLT + kMaxHalves * kHalf * 32;  // 149 KiB
 static_assert(2 * kT * kTokBytes == kStagesBytes && kOffC == kStageBytes,
               "the B and C tiles are the GEMM's two stages");
 static_assert(kLdsFused <= 160 * 1024, "gfx950 LDS");
+
+using WRows = WRowsOf<4 * kHalf>;  // half of the tile's 256 rows from each weight
 
 // 16-bit tensors (bf16 or fp16, the kernel's T) as raw element bits.
 struct FusedArgs {
@@ -96,24 +95,7 @@ struct FusedArgs {
 // 256-byte row, so the 16 tokens one epilogue store instruction writes spread over the
 // banks, while the 32 states one walk read takes stay one contiguous row.
 
-// Rows of one K stage for the GEMM tile of (time tile, half): W rows [0, 128) from
-// W_B and [128, 256) from W_C, the half's 4 hs rows each (rows past them read the
-// half's first state: in a ragged last half the 8-row groups of a DMA instruction are
-// whole pairs of states, d_state being even); X rows the tile's tv tokens (rows past
-// the sequence read its last token).
-struct WRows {
-  const uint16_t* wb;
-  const uint16_t* wc;
-  int64_t row0;
-  int hs4, K;
-  __device__ const void* operator()(int g, int k0, int i, uint32_t& voff,
-                                    const DmaLane& dl) const {
-    voff = (uint32_t)(dl.lrow * K * 2) + dl.cb(i);
-    const int r = g & 127;  // 8-row groups never straddle B and C
-    const int rr = r < hs4 ? r : 0;
-    return (g < 128 ? wb : wc) + ((row0 + rr) * K + k0);
-  }
-};
+// X rows of one K stage: the tile's tv tokens (rows past the sequence read its last token).
 template <bool FULL_T>
 struct XRows {
   const uint16_t* x;
@@ -131,53 +113,6 @@ struct XRows {
     return x + ((row0 + gb) * K + k0);
   }
 };
-
-// The walk's and the epilogue's LDS addresses are the same for every tile; left to
-// itself the compiler computes them once and holds them (tens of registers) through
-// the K loop, which then spills. Passing a lane's base through this empty statement
-// makes it opaque, so the addresses derived from it are recomputed where used.
-template <typename V>
-__device__ inline V opaque(V v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-
-// The two 16-bit elements of a 32-bit word (low half first) in fp32.
-template <typename T>
-__device__ inline float lo16(uint32_t w) {
-  if constexpr (std::is_same<T, bf16_t>::value) return __uint_as_float(w << 16);
-  else return io<T>::bits_to_f32(w & 0xffffu);
-}
-template <typename T>
-__device__ inline float hi16(uint32_t w) {
-  if constexpr (std::is_same<T, bf16_t>::value) return __uint_as_float(w & 0xffff0000u);
-  else return io<T>::bits_to_f32(w >> 16);
-}
-
-// Exchange x of the odd 16-lane rows with y of the even rows (v_permlane16_swap_b32):
-// afterwards even-row lanes hold (own x, the odd neighbour's x) and odd-row lanes
-// (the even neighbour's y, own y). Issued as assembly with both registers read-write,
-// as the library's other row swaps (common.hpp), N pairs behind one pair of s_nops.
-template <int N>
-__device__ inline void row_swap16(float* x, float* y) {
-  static_assert(N == 8, "eight pairs per statement");
-  asm volatile(
-      "s_nop 1\n\t"
-      "v_permlane16_swap_b32 %0, %8\n\t"
-      "v_permlane16_swap_b32 %1, %9\n\t"
-      "v_permlane16_swap_b32 %2, %10\n\t"
-      "v_permlane16_swap_b32 %3, %11\n\t"
-      "v_permlane16_swap_b32 %4, %12\n\t"
-      "v_permlane16_swap_b32 %5, %13\n\t"
-      "v_permlane16_swap_b32 %6, %14\n\t"
-      "v_permlane16_swap_b32 %7, %15\n\t"
-      "s_nop 1"
-      : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]),
-        "+v"(x[7]), "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]),
-        "+v"(y[6]), "+v"(y[7]));
-}
-
-__device__ inline float row_half_mirror(float v) { return dpp_mov<0x141>(v); }
 
 // Sum of o[64] (16 tokens x 4 components of one chunk, i = 4 j + comp) over the 32 lanes
 // of each half-wave, scattered: lane u (= lane & 31) ends with the sums of indices

@@ -169,7 +169,6 @@ __device__ inline void tile_issue_stage(int kt, int wave, uint32_t lds0, const D
   }
 }
 
-//
 // SPLIT: each row holds an fp32 row as two fp16 pieces (gemm_f32.hip), a K step's 128 bytes
 // being 32 columns' high pieces and then the same columns' low pieces, so the two "K slices"
 // of a step are W_hi, W_lo and X_hi, X_lo, and the step's products are W_hi X_hi, W_hi X_lo
@@ -242,6 +241,105 @@ __device__ inline void tile_kloop_cfg(int K, char* lds,
     } else {
       mfmas(1, 1);
     }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// The K loop for tiles whose weights stream from HBM: NSW LDS slots for W and NSX for X (the W
+// slots first), so NSW - 1 stages of weights are in flight while one is multiplied; X, which the
+// L2 holds, may have fewer slots. The caller has issued W stages 0 .. NSW - 2 and X stages 0 ..
+// NSX - 2 (tile_issue_w, tile_issue_x), those of a stage together, X last, and loaded nothing since that it has not waited for.
+template <typename Cfg, int NSW, typename WRow>
+__device__ inline void tile_issue_w(int kt, int slot, int wave, uint32_t lds0, const DmaLane& dl,
+                                    const WRow& wrow) {
+#pragma unroll
+  for (int i = 0; i < Cfg::kWLoads; ++i) {
+    const int gi = wave * Cfg::kWLoads + i;
+    uint32_t v;
+    const void* b = wrow(gi * kRowsPerLoad, kt * kBK, gi, v, dl);
+    dma16(b, v, lds0 + (uint32_t)(slot * Cfg::kWBytes + gi * 1024));
+  }
+}
+template <typename Cfg, int NSW, typename XRow>
+__device__ inline void tile_issue_x(int kt, int slot, int wave, uint32_t lds0, const DmaLane& dl,
+                                    const XRow& xrow) {
+  constexpr int kXBytes = Cfg::TX * kRowBytes;
+#pragma unroll
+  for (int i = 0; i < Cfg::kXLoads; ++i) {
+    const int gi = wave * Cfg::kXLoads + i;
+    uint32_t v;
+    const void* b = xrow(gi * kRowsPerLoad, kt * kBK, gi, v, dl);
+    dma16(b, v, lds0 + (uint32_t)(NSW * Cfg::kWBytes + slot * kXBytes + gi * 1024));
+  }
+}
+
+template <typename Cfg, int NSW, int NSX, typename E, typename WRow, typename XRow>
+__device__ inline void tile_kloop_deep(int K, char* lds, floatx4 (&acc)[Cfg::WB][Cfg::XB],
+                                       const WRow& wrow, const XRow& xrow) {
+  static_assert(NSX == 2 || NSX == NSW, "the waits below");
+  constexpr int WB = Cfg::WB, XB = Cfg::XB;
+  constexpr int kXBytes = Cfg::TX * kRowBytes;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const DmaLane dl(lane);
+  const uint32_t lds0 = lds_addr(lds);
+  const int wn = wave / Cfg::NW_X;
+  const int wm = wave % Cfg::NW_X;
+  const int rl = lane & 15;
+  const int q = lane >> 4;
+  int woff[2], xoff[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int c = 4 * kk + q;
+    const int rw = wn * (Cfg::TW / Cfg::NW_W) + rl;
+    woff[kk] = rw * kRowBytes + gswz(rw, c) * 16;
+    const int rx = wm * (Cfg::TX / Cfg::NW_X) + rl;
+    xoff[kk] = NSW * Cfg::kWBytes + rx * kRowBytes + gswz(rx, c) * 16;
+  }
+  using frag = typename FragOf<E>::type;
+  const int KT = K / kBK;
+  int ws = 0, xs = 0;
+  for (int kt = 0; kt < KT; ++kt) {
+    // Loads return in order. Issued after this step's X (the last of its stage to go out):
+    // with as many X slots as W slots NSW - 2 whole stages, with two the W stage issued
+    // beside it. (Towards the end there are fewer, and all are waited for.)
+    if (kt + NSW - 2 < KT)
+      wait_vmcnt<NSX == 2 ? (NSW > 2 ? Cfg::kWLoads : 0)
+                          : (NSW - 2) * (Cfg::kWLoads + Cfg::kXLoads)>();
+    else
+      wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    // The slots consumed before the barrier are free.
+    const int wfree = ws == 0 ? NSW - 1 : ws - 1, xfree = xs == 0 ? NSX - 1 : xs - 1;
+    if constexpr (NSX == 2) {
+      if (kt + 1 < KT) tile_issue_x<Cfg, NSW>(kt + 1, xfree, wave, lds0, dl, xrow);
+      if (kt + NSW - 1 < KT) tile_issue_w<Cfg, NSW>(kt + NSW - 1, wfree, wave, lds0, dl, wrow);
+    } else if (kt + NSW - 1 < KT) {
+      tile_issue_w<Cfg, NSW>(kt + NSW - 1, wfree, wave, lds0, dl, wrow);
+      tile_issue_x<Cfg, NSW>(kt + NSW - 1, xfree, wave, lds0, dl, xrow);
+    }
+    const char* wb = lds + ws * Cfg::kWBytes;
+    const char* xb = lds + xs * kXBytes;
+    ws = ws == NSW - 1 ? 0 : ws + 1;
+    xs = xs == NSX - 1 ? 0 : xs + 1;
+    frag wf[2][WB], xf[2][XB];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int nb = 0; nb < WB; ++nb)
+        wf[kk][nb] = *(const frag*)(wb + woff[kk] + nb * 16 * kRowBytes);
+#pragma unroll
+      for (int mb = 0; mb < XB; ++mb)
+        xf[kk][mb] = *(const frag*)(xb + xoff[kk] + mb * 16 * kRowBytes);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int nb = 0; nb < WB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < XB; ++mb)
+          acc[nb][mb] = mfma16(wf[kk][nb], xf[kk][mb], acc[nb][mb]);
     __builtin_amdgcn_sched_barrier(0);
   }
 }

@@ -263,14 +263,18 @@ struct LamConst {
   float a, n2, v0, v1, v2;
 };
 
-__device__ inline LamConst lam_const(const float* lam_alpha, const float* lam_imag, int64_t dk) {
+__device__ inline LamConst lam_from(float alpha, float i0, float i1, float i2) {
   LamConst c;
-  c.a = -softplus_f(lam_alpha[dk]);
-  c.v0 = tanhf(lam_imag[dk * 3 + 0]);
-  c.v1 = tanhf(lam_imag[dk * 3 + 1]);
-  c.v2 = tanhf(lam_imag[dk * 3 + 2]);
+  c.a = -softplus_f(alpha);
+  c.v0 = tanhf(i0);
+  c.v1 = tanhf(i1);
+  c.v2 = tanhf(i2);
   c.n2 = 0.25f * (c.a * c.a + c.v0 * c.v0 + c.v1 * c.v1 + c.v2 * c.v2);
   return c;
+}
+
+__device__ inline LamConst lam_const(const float* lam_alpha, const float* lam_imag, int64_t dk) {
+  return lam_from(lam_alpha[dk], lam_imag[dk * 3 + 0], lam_imag[dk * 3 + 1], lam_imag[dk * 3 + 2]);
 }
 
 // q = Cayley(dl * Lambda) = ((1 - dl^2 n2) / N, dl v / N), N = max(1 - dl a + dl^2 n2, eps).

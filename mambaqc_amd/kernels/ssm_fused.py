@@ -495,6 +495,32 @@ FUSED_BC_SPLIT_MAX_BATCH = 1
 # segments of time, the state carried from one to the next through h0 / h_last.
 FUSED_BC_SPLIT_WS_MAX = 4 << 30
 
+# Sequences of up to this many tokens run in tiles of 64 or 128 tokens
+# (mqc_ssm_fused_bc_short_fwd) instead of the 256-token tile: d_inner 1536, 64 states, batch 1,
+# 100 tokens 514 us against 646, d_inner 1024, 32 states 118 against 157.
+FUSED_BC_SHORT_MAX_SEQ = 128
+# Against the projections by themselves and the walk (us, bf16). While one tile holds the whole
+# batch every weight row is read once, and the short form is the faster one: d_inner 1536, 64
+# states, batch 1 x 17 tokens 410 / 503, x 64 454 / 572, x 100 514 / 633, x 128 544 / 656,
+# 2 x 64 539 / 632; d_inner 512 x 64 states 1 x 100 66 / 117. Several tiles each stream the weights
+# through L2 again where the GEMM shares them: 2 x 100 788 / 666, 4 x 64 812 / 686, and at d_inner 1024,
+# 32 states (512 MiB of weights) 191 / 201 and 194 / 196. Weights that fit the Infinity Cache together
+# still win: d_inner 512, 64 states (256 MiB) 4 x 64 115 / 140, 4 x 100 223 / 218, 4 x 128 227 / 267;
+# 16 states 4 x 128 59 / 92. Up to 16 rows the decode projections (skinny GEMM) stream the weights at HBM speed
+# already.
+FUSED_BC_SHORT_MIN_ROWS = 17
+FUSED_BC_SHORT_CACHED_BYTES = 256 << 20
+
+
+def fused_bc_short_wins(batch: int, seq_len: int, d_inner: int, d_state: int) -> bool:
+    """Whether the fused short form beats separate projections for these sizes (of at most
+    FUSED_BC_SHORT_MAX_SEQ tokens; 16-bit operands)."""
+    if not 0 < seq_len <= FUSED_BC_SHORT_MAX_SEQ or batch * seq_len < FUSED_BC_SHORT_MIN_ROWS:
+        return False
+    one_tile = batch * (-(-seq_len // 8) * 8) <= 128
+    return one_tile or 2 * d_inner * d_state * 4 * d_inner * 2 <= FUSED_BC_SHORT_CACHED_BYTES
+
+
 def fused_bc_eligible(x: torch.Tensor, B_weight: torch.Tensor, C_weight: torch.Tensor,
                       d_state: int, dtype: torch.dtype | None = None) -> bool:
     """Whether ssm_forward_fused_bc takes these operands: x [batch, T, d_inner] with
@@ -531,7 +557,8 @@ def ssm_forward_fused_bc(x: torch.Tensor, B_weight: torch.Tensor, C_weight: torc
     return_state). Inference only (no autograd).
     split: run each half of the states (32) in a workgroup of its own, with a
     workspace for the halves' partial sums and a second launch adding them (the
-    same y bit for bit); None splits batches of at most FUSED_BC_SPLIT_MAX_BATCH.
+    same y bit for bit); None splits batches of at most FUSED_BC_SPLIT_MAX_BATCH, and
+    runs sequences of at most FUSED_BC_SHORT_MAX_SEQ tokens in the short form.
     """
     batch, T, d_inner = x.shape
     d_state = lambda_alpha.shape[-1] if lambda_alpha.dim() == 2 else 0
@@ -563,9 +590,17 @@ def ssm_forward_fused_bc(x: torch.Tensor, B_weight: torch.Tensor, C_weight: torc
     code = nat.dtype_code(xc)
     h_last = (torch.empty(batch, d_inner, d_state, 4, device=x.device, dtype=torch.float32)
               if return_state else None)
+    lib = nat.load()
+    if split is None and 0 < T <= FUSED_BC_SHORT_MAX_SEQ:
+        ws_bytes = lib.mqc_ssm_fused_bc_short_workspace_bytes(batch, T, d_inner, d_state)
+        ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8) if ws_bytes else None
+        nat.call("mqc_ssm_fused_bc_short_fwd", xc, xc.data_ptr(), wb.data_ptr(), wc.data_ptr(),
+                 dl.data_ptr(), sv.data_ptr(), la.data_ptr(), li.data_ptr(), Dv.data_ptr(),
+                 nat.ptr(h0c), y.data_ptr(), nat.ptr(h_last), batch, T, d_inner, d_state,
+                 float(eps), code, nat.ptr(ws), ws_bytes, nat.stream_of(xc))
+        return (y, h_last) if return_state else y
     if split is None:
         split = batch <= FUSED_BC_SPLIT_MAX_BATCH
-    lib = nat.load()
     ws_bytes = lib.mqc_ssm_fused_bc_split_workspace_bytes(batch, T, d_inner, d_state) if split else 0
     stream = nat.stream_of(xc)
     if ws_bytes <= 0:
