@@ -39,6 +39,39 @@ int mqc_ssm_fused_bc_short_fwd(const void* x, const void* B_weight, const void* 
                                int64_t d_state, float eps, int dtype, void* workspace,
                                int64_t workspace_bytes, void* stream);
 
+/* One recurrent decode step of the block in four launches (bf16 or fp16; M = batch, 1 to 16
+ * rows, K and 4 d_inner multiples of 32, X within the skinny GEMM's 64 KiB of LDS, else
+ * MQC_E_LIMIT). Each rounds to dtype where the separate launches store.
+ *
+ * mqc_step_in_proj_conv: X [M, K] times W [>= channels + z_cols, K] (+ bias); the first
+ * `channels` columns are one step of mqc_causal_conv_silu_step (continued from and shifting
+ * tail [M, conv_k - 1, channels]) into act [M, channels], the next z_cols go to z [M, z_cols].
+ * channels a multiple of 8, conv_k at most 4.
+ * mqc_gemm_skinny4_nt: mqc_gemm_skinny_nt for four weights sharing X.
+ * mqc_step_ssm: delta = softplus(dt_raw), s = sigmoid(g_raw) x, then one step of
+ * mqc_ssm_fused_fwd in place on h (fp32 [batch, d_inner, d_state, 4]); d_state <= 64.
+ * mqc_step_norm_out_gate: mqc_qln_fwd of Y [M, d_inner, 4], times W [d_model, 4 d_inner]
+ * (+ bias), out = x + sigmoid(z) * that (x, out [M, d_model]; z rows z_row_stride apart). */
+int mqc_step_in_proj_conv(const void* X, int64_t M, int64_t K, const void* W, const void* bias,
+                          int64_t channels, int64_t z_cols, const float* conv_w,
+                          const float* conv_b, int64_t conv_k, void* tail, void* act, void* z,
+                          int dtype, void* stream);
+int mqc_gemm_skinny4_nt(const void* X, int64_t M, int64_t K, const void* W1, const void* bias1,
+                        void* Y1, int64_t N1, const void* W2, const void* bias2, void* Y2,
+                        int64_t N2, const void* W3, const void* bias3, void* Y3, int64_t N3,
+                        const void* W4, const void* bias4, void* Y4, int64_t N4, int dtype,
+                        void* stream);
+int mqc_step_ssm(const void* dt_raw, const void* g_raw, const void* x, const void* B,
+                 const void* C, const float* lambda_alpha, const float* lambda_imag,
+                 const float* D, float* h, void* y, int64_t batch, int64_t d_inner,
+                 int64_t d_state, float eps, int dtype, void* stream);
+int mqc_step_norm_out_gate(const void* Y, int64_t M, int64_t d_inner, const float* gamma,
+                           const float* beta, float eps, const void* W, const void* bias,
+                           int64_t d_model, const void* x, const void* z, int64_t z_row_stride,
+                           void* out, int dtype, void* stream);
+/* 1 where mqc_step_norm_out_gate takes M rows of d_inner quaternions, else 0. */
+int mqc_step_norm_out_gate_fits(int64_t M, int64_t d_inner);
+
 #ifdef __cplusplus
 }
 #endif

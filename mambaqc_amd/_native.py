@@ -92,6 +92,14 @@ SIGNATURES_EXT = {
                      _vp],
     "mqc_ssm_fused_bc_short_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                    _i64, _i64, _i64, _i64, _f32, _int, _vp, _i64, _vp],
+    "mqc_gemm_skinny4_nt": [_vp, _i64, _i64] + [_vp, _vp, _vp, _i64] * 4 + [_int, _vp],
+    "mqc_step_in_proj_conv": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp,
+                              _int, _vp],
+    "mqc_step_norm_out_gate": [_vp, _i64, _i64, _vp, _vp, _f32, _vp, _vp, _i64, _vp, _vp, _i64,
+                               _vp, _int, _vp],
+    "mqc_step_norm_out_gate_fits": [_i64, _i64],
+    "mqc_step_ssm": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32,
+                     _int, _vp],
 }
 SIGNATURES_EXT_I64 = {
     "mqc_ssm_fused_bc_short_workspace_bytes": [_i64, _i64, _i64, _i64],

@@ -43,7 +43,7 @@ from .kernels.ssm_fused import (fused_bc_eligible, ssm_forward_front_dl, ssm_for
                                 ssm_forward_fused_dl, ssm_front)
 from .layers.causal_conv1d import CausalConv1d, causal_conv1d_silu, causal_conv1d_silu_step_
 from .layers.quaternion_linear import (quaternion_to_real_projection, real_to_quaternion_projection,
-                                      skinny_eligible, skinny_linear)
+                                      skinny_eligible, skinny_linear, skinny_shape_eligible)
 
 
 def _gate_operands(x, z, y_real):
@@ -455,6 +455,17 @@ class QuaternionMamba2Block(nn.Module):
         Feeding a sequence in pieces gives the same outputs as feeding it whole
         (up to rounding), which is what recurrent decoding relies on.
         """
+        b, t, _ = x.shape
+        if t == 1 and self._step_fused_ok(x):
+            # One token: the decode step, on copies of the state.
+            if state is None:
+                tail = x.new_zeros(b, self.d_conv - 1, self.d_inner)
+                h = x.new_zeros(b, self.d_inner, self.d_state, 4, dtype=torch.float32)
+            else:
+                tail = state[0].to(x.dtype).clone(memory_format=torch.contiguous_format)
+                h = state[1].to(torch.float32).clone(memory_format=torch.contiguous_format)
+            if self._step_state_ok(x, tail, h):
+                return self._step_fused(x, tail, h), (tail, h)
         xz = _linear(self.in_proj, x)
         x_in, z = xz.chunk(2, dim=-1)
         b, _, D = x_in.shape
@@ -482,6 +493,8 @@ class QuaternionMamba2Block(nn.Module):
         kernel that also shifts it, and the SSM writes its final state over h, so
         the step copies no state."""
         tail, h = state
+        if self._step_fused_ok(x) and self._step_state_ok(x, tail, h):
+            return self._step_fused(x, tail, h)
         xz = _linear(self.in_proj, x)
         x_in, z = xz.chunk(2, dim=-1)
         conv = self.conv1d.conv
@@ -492,6 +505,84 @@ class QuaternionMamba2Block(nn.Module):
                                             self.Lambda_imag, self.D, h, eps=1e-6)
         y_real = _out_proj(self.out_proj, self.norm(y))
         return out_gate(x, z, y_real)
+
+    def _step_fused_ok(self, x: torch.Tensor) -> bool:
+        """Whether one token per sequence of x runs as the four launches of _step_fused: 16-bit,
+        no autograd, autocast or compilation, decode-sized weights, the block's own LayerNorm
+        without hooks."""
+        D, dm = self.d_inner, self.d_model
+        if (nat.compiling() or not x.is_cuda or x.dim() != 3 or x.shape[1] != 1
+                or x.shape[2] != dm or self.d_state > 64 or self.d_conv > 4 or D % 8):
+            return False
+        rows = x.shape[0]
+        ip, op, conv, norm = self.in_proj, self.out_proj, self.conv1d.conv, self.norm
+        flat = lambda b: None if b is None else b.reshape(-1)  # noqa: E731
+        others = (self.Lambda_alpha, self.Lambda_imag, self.D, conv.weight, conv.bias,
+                  norm.gamma, norm.beta)
+        if torch.is_grad_enabled() and any(p is not None and p.requires_grad for p in others):
+            return False
+        return (type(norm) is QuaternionLayerNorm
+                and not norm._forward_hooks and not norm._forward_pre_hooks
+                and all(p is None or p.device == x.device for p in others)
+                and skinny_shape_eligible(x, rows, dm, ip.weight, ip.bias)
+                and skinny_shape_eligible(
+                    x, rows, D, self.dt_proj.weight, self.dt_proj.bias, self.gate_proj.weight,
+                    self.gate_proj.bias, self.B_proj.weight, flat(self.B_proj.bias),
+                    self.C_proj.weight, flat(self.C_proj.bias)))
+
+    def _step_state_ok(self, x: torch.Tensor, tail: torch.Tensor, h: torch.Tensor) -> bool:
+        """A recurrent state that the fused step takes in place (any other goes through the
+        separate launches, and their checks)."""
+        b = x.shape[0]
+        return (tail.shape == (b, self.d_conv - 1, self.d_inner) and tail.dtype == x.dtype
+                and tail.is_contiguous() and tail.device == x.device
+                and h.shape == (b, self.d_inner, self.d_state, 4) and h.dtype == torch.float32
+                and h.is_contiguous() and h.data_ptr() % 16 == 0 and h.device == x.device
+                and not (torch.is_grad_enabled() and (tail.requires_grad or h.requires_grad)))
+
+    def _step_fused(self, x: torch.Tensor, tail: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
+        """step_state_ in four launches where the separate steps take nine (each about 4 us of a
+        captured step): [in_proj, of the gate half only the columns that the gate reads, + conv],
+        [dt, gate, B and C projections], [front + SSM step], [LayerNorm + out_proj + gate and
+        residual]. The last falls back to three launches where the LayerNorm's rows do not fit
+        that kernel. Base preset's block, 4 sequences 426 -> 413 us (384 of them B and C's weights);
+        small preset's whole decode step as a graph 980 -> 899 us."""
+        b, D, S, dm = x.shape[0], self.d_inner, self.d_state, self.d_model
+        new = lambda *shape: torch.empty(*shape, device=x.device, dtype=x.dtype)  # noqa: E731
+        code, stream = nat.dtype_code(x), nat.stream_of(x)
+        xc = nat.aligned16(x.detach())
+        ip, conv, op = self.in_proj, self.conv1d.conv, self.out_proj
+        act, z = new(b, 1, D), new(b, 1, dm)
+        cw = nat.param_f32(conv.weight)
+        cb = None if conv.bias is None else nat.param_f32(conv.bias)
+        nat.call("mqc_step_in_proj_conv", xc, xc.data_ptr(), b, dm, ip.weight.data_ptr(),
+                 nat.ptr(ip.bias), D, dm, cw.data_ptr(), nat.ptr(cb), self.d_conv,
+                 tail.data_ptr(), act.data_ptr(), z.data_ptr(), code, stream)
+        dt, g = new(b, 1, D), new(b, 1, D)
+        Bq, Cq = new(b, 1, D, S, 4), new(b, 1, D, S, 4)
+        args = []
+        for layer, y in ((self.dt_proj, dt), (self.gate_proj, g), (self.B_proj, Bq),
+                         (self.C_proj, Cq)):
+            args += [layer.weight.data_ptr(), nat.ptr(layer.bias), y.data_ptr(),
+                     layer.weight.shape[0]]
+        nat.call("mqc_gemm_skinny4_nt", act, act.data_ptr(), b, D, *args, code, stream)
+        la, li, Dv = (nat.param_f32(p) for p in (self.Lambda_alpha, self.Lambda_imag, self.D))
+        y = new(b, 1, D, 4)
+        nat.call("mqc_step_ssm", act, dt.data_ptr(), g.data_ptr(), act.data_ptr(), Bq.data_ptr(),
+                 Cq.data_ptr(), la.data_ptr(), li.data_ptr(), Dv.data_ptr(), h.data_ptr(),
+                 y.data_ptr(), b, D, S, 1e-6, code, stream)
+        w, ob = op.weight, op.bias
+        if not (nat.load().mqc_step_norm_out_gate_fits(b, D) and w.dtype == x.dtype
+                and w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and (ob is None or (ob.dtype == x.dtype and ob.is_contiguous()))
+                and not (torch.is_grad_enabled() and w.requires_grad)):
+            return out_gate(x, z, _out_proj(op, self.norm(y)))
+        gamma, beta = nat.param_f32(self.norm.gamma), nat.param_f32(self.norm.beta)
+        out = new(b, 1, dm)
+        nat.call("mqc_step_norm_out_gate", y, y.data_ptr(), b, D, gamma.data_ptr(),
+                 beta.data_ptr(), float(self.norm.eps), w.data_ptr(), nat.ptr(ob), dm,
+                 xc.data_ptr(), z.data_ptr(), dm, out.data_ptr(), code, stream)
+        return out
 
     def _ssm_forward(self, x: torch.Tensor, h0: torch.Tensor | None = None,
                      return_state: bool = False):

@@ -233,6 +233,24 @@ __device__ inline float sum_halves_to_low(float v) {
 }
 
 // ---------------------------------------------------------------------------
+// The SSM's front (elementwise.hip; the decode step): delta = softplus(dt_raw) and the gate's
+// sigmoid.
+// ---------------------------------------------------------------------------
+// softplus(v) = max(v, 0) + log(1 + e) with e = exp(-|v|) in (0, 1]; for e < 1e-2
+// the log comes from its series (four terms), so the relative error stays below
+// 1e-5 also where softplus(v) ~ exp(v) is tiny (6e-6 worst case in an fp32
+// emulation over [-40, 25]). The hardware exp/log/reciprocal (about 1 ulp) keep
+// the kernel at HBM speed.
+__device__ inline float front_softplus(float v) {
+  if (v > 20.f) return v;
+  const float e = __expf(-fabsf(v));
+  const float l = e < 1e-2f ? e * (1.f - e * (0.5f - e * (1.f / 3.f - 0.25f * e)))
+                            : __logf(1.f + e);
+  return fmaxf(v, 0.f) + l;
+}
+__device__ inline float front_sigmoid(float v) { return __builtin_amdgcn_rcpf(1.f + __expf(-v)); }
+
+// ---------------------------------------------------------------------------
 // XCD-aware block order. MI355X dispatches the workgroups of a launch to its 8
 // XCDs (each with its own L2) round-robin by linear block id, so neighbouring
 // blocks land on different L2s. Where neighbouring blocks share cache lines

@@ -283,20 +283,6 @@ int launch_out_gate_bwd(const void* dout, const void* z, int64_t zs, const void*
 //   d_dt_raw = d_delta * sigmoid(dt_raw)   (1 above the threshold)
 //   d_g_raw  = d_s * x * sig(g) * (1 - sig(g)),   d_x = d_s * sig(g)
 // ---------------------------------------------------------------------------
-// softplus(v) = max(v, 0) + log(1 + e) with e = exp(-|v|) in (0, 1]; for e < 1e-2
-// the log comes from its series (four terms), so the relative error stays below
-// 1e-5 also where softplus(v) ~ exp(v) is tiny (6e-6 worst case in an fp32
-// emulation over [-40, 25]). The hardware exp/log/reciprocal (about 1 ulp) keep
-// the kernel at HBM speed.
-__device__ inline float front_softplus(float v) {
-  if (v > 20.f) return v;
-  const float e = __expf(-fabsf(v));
-  const float l = e < 1e-2f ? e * (1.f - e * (0.5f - e * (1.f / 3.f - 0.25f * e)))
-                            : __logf(1.f + e);
-  return fmaxf(v, 0.f) + l;
-}
-__device__ inline float front_sigmoid(float v) { return __builtin_amdgcn_rcpf(1.f + __expf(-v)); }
-
 template <typename T, int V>
 __global__ __launch_bounds__(kThreads) void ssm_front_kernel(const T* __restrict__ dt,
                                                              const T* __restrict__ g,

@@ -261,6 +261,7 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 # of [1024 x 1024] weights 6.3 us in one launch against about 6.6 us per weight
 # through hipBLASLt, [131072 x 1024] pairs 95-98 against 99.7 us.
 SKINNY_MAX_ROWS = 16
+SKINNY_MAX_LDS = 64 << 10  # the rows of X, each padded by 16 bytes
 # With at most SKINNY_WIDE_MAX_ROWS token rows and K a multiple of 64, the
 # library streams large weights in its wide mode (whole 128-byte lines per load,
 # VALU dot products), faster than hipBLASLt's GEMV: the base preset's
@@ -286,16 +287,21 @@ def skinny_eligible(x: torch.Tensor, *params) -> bool:
     dtype, K a multiple of 32, dense weights (of at most SKINNY_MAX_WEIGHT_BYTES
     unless the wide mode applies), nothing recording autograd, no autocast, not
     under torch.compile."""
+    K = x.shape[-1] if x.dim() else 0
+    return skinny_shape_eligible(x, x.numel() // K if K else 0, K, *params)
+
+
+def skinny_shape_eligible(x: torch.Tensor, rows: int, K: int, *params) -> bool:
+    """skinny_eligible for an input of `rows` rows of K computed from x (its device, dtype and
+    autograd state)."""
     if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or x.dim() < 1:
         return False
-    K = x.shape[-1]
-    rows = x.numel() // K if K else 0
-    if not (0 < rows <= SKINNY_MAX_ROWS) or K % 32 or rows * (K + 8) * 2 > (64 << 10):
+    if not (0 < rows <= SKINNY_MAX_ROWS) or K % 32 or rows * (K + 8) * 2 > SKINNY_MAX_LDS:
         return False
     if torch.compiler.is_compiling() or torch.is_autocast_enabled(x.device.type):
         return False
-    tensors = [x] + [p for p in params if p is not None]
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+    if torch.is_grad_enabled() and (x.requires_grad or any(
+            p is not None and p.requires_grad for p in params)):
         return False
     wide = _skinny_wide(rows, K)
     for w, b in zip(params[0::2], params[1::2]):
