@@ -25,6 +25,11 @@ int mqc_gemm_f32(const float* X, int64_t x_row, int64_t x_col, const float* W, i
                  int64_t w_col, float* Y, int64_t ldy, int64_t M, int64_t N, int64_t K,
                  void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Up to four small fp32 products in one launch, Y[m * N + n] = sum_k X[m * xm + k * xk] *
+ * W[n * wn + k * wk] (+ bias[n]). products: count rows of eleven values, X, xm, xk, W, wn, wk,
+ * bias (or 0), Y, M, N, K (pointers as integers; one of xm, xk and one of wn, wk is 1). */
+int mqc_gemm_f32_small(const int64_t* products, int64_t count, void* stream);
+
 /* mqc_ssm_fused_bc_fwd for short sequences, seq_len from 1 to 128 (MQC_E_LIMIT above): same
  * operands, dtypes, shapes and refusals, in tiles of 64 or 128 tokens that hold whole
  * sequences of the batch, each group of 16 states in a workgroup of its own. d_state > 16

@@ -92,6 +92,7 @@ SIGNATURES_EXT = {
                      _vp],
     "mqc_ssm_fused_bc_short_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                    _i64, _i64, _i64, _i64, _f32, _int, _vp, _i64, _vp],
+    "mqc_gemm_f32_small": [_vp, _i64, _vp],
     "mqc_gemm_skinny4_nt": [_vp, _i64, _i64] + [_vp, _vp, _vp, _i64] * 4 + [_int, _vp],
     "mqc_step_in_proj_conv": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp,
                               _int, _vp],
@@ -185,8 +186,17 @@ def compiling() -> bool:
     return torch.compiler.is_compiling()
 
 
+# The raw forms of torch.cuda.current_stream(device).cuda_stream and current_device(): a call's
+# host time is what bounds small blocks, and the public ones build a Stream object per call
+# (4.5 us against 0.3).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -233,15 +243,21 @@ def param_f32(t: torch.Tensor) -> torch.Tensor:
     return conv
 
 
+_fns: dict = {}
+
+
 def call(name: str, device_tensor: torch.Tensor, *args) -> None:
     """Call entry point `name` with the tensor's device current (the library
     launches on the device that is current; the stream argument must belong to
     it). The device switch is skipped when it is current already."""
-    fn = getattr(load(), name)
-    idx = device_tensor.device.index
-    if idx is None or idx == torch.cuda.current_device():
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns.setdefault(name, getattr(load(), name))
+    idx = device_tensor.get_device()
+    if idx == (_raw_device() if _raw_device is not None else torch.cuda.current_device()):
         status = fn(*args)
     else:
         with torch.cuda.device(idx):
             status = fn(*args)
-    check(status, name)
+    if status != 0:
+        check(status, name)

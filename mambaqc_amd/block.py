@@ -42,8 +42,10 @@ from .kernels import ssm_fused as _sf
 from .kernels.ssm_fused import (fused_bc_eligible, ssm_forward_front_dl, ssm_forward_fused_bc,
                                 ssm_forward_fused_dl, ssm_front)
 from .layers.causal_conv1d import CausalConv1d, causal_conv1d_silu, causal_conv1d_silu_step_
-from .layers.quaternion_linear import (quaternion_to_real_projection, real_to_quaternion_projection,
-                                      skinny_eligible, skinny_linear, skinny_shape_eligible)
+from .layers.quaternion_linear import (QuaternionLinear, quaternion_to_real_projection,
+                                      real_to_quaternion_projection,
+                                      f32_small_eligible, f32_small_linears, skinny_eligible,
+                                      skinny_linear, skinny_shape_eligible)
 
 
 def _gate_operands(x, z, y_real):
@@ -221,10 +223,26 @@ def bc_slice_width(batch: int, seq_len: int, d_inner: int, d_state: int, elsize:
     return max(1, min(d_inner, budget // max(per_d, 1)))
 
 
+def _unhooked(*layers: nn.Module) -> bool:
+    """Plain nn.Linear layers without hooks, whose call is F.linear and nothing more."""
+    return all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks
+                                             or m._backward_hooks or m._backward_pre_hooks)
+               for m in layers)
+
+
+def _unhooked_quaternion(*layers) -> bool:
+    return all(type(m) is QuaternionLinear and not (m._forward_hooks or m._forward_pre_hooks
+                                                    or m._backward_hooks or m._backward_pre_hooks)
+               for m in layers)
+
+
 def _linear(layer: nn.Linear, x: torch.Tensor) -> torch.Tensor:
-    """layer(x), on the library's skinny GEMM for decode-sized inputs."""
+    """layer(x), on the library's skinny GEMM for decode-sized inputs and its small GEMM for
+    small fp32 ones."""
     if skinny_eligible(x, layer.weight, layer.bias):
         return skinny_linear(x, layer.weight, layer.bias)
+    if _unhooked(layer) and f32_small_eligible(x, layer.weight, layer.bias):
+        return f32_small_linears(x, layer.weight, layer.bias)[0]
     return layer(x)
 
 
@@ -232,6 +250,8 @@ def _linear_pair(a: nn.Linear, b: nn.Linear, x: torch.Tensor):
     """(a(x), b(x)), in one skinny launch for decode-sized inputs."""
     if skinny_eligible(x, a.weight, a.bias, b.weight, b.bias):
         return skinny_linear(x, a.weight, a.bias, b.weight, b.bias)
+    if _unhooked(a, b) and f32_small_eligible(x, a.weight, a.bias, b.weight, b.bias):
+        return f32_small_linears(x, a.weight, a.bias, b.weight, b.bias)
     return a(x), b(x)
 
 
@@ -592,7 +612,18 @@ class QuaternionMamba2Block(nn.Module):
             x.requires_grad or (h0 is not None and h0.requires_grad)
             or any(p.requires_grad for p in self.parameters()))
         width = self._bc_slice_width(x, recording)
-        dt_raw, g_raw = _linear_pair(self.dt_proj, self.gate_proj, x)
+        dtp, gp, bp, cp = self.dt_proj, self.gate_proj, self.B_proj, self.C_proj
+        Bq = Cq = None
+        if (not recording and not width and bp.bias is None and cp.bias is None
+                and _unhooked(dtp, gp) and _unhooked_quaternion(bp, cp)
+                and f32_small_eligible(x, dtp.weight, dtp.bias, gp.weight, gp.bias,
+                                       bp.weight, None, cp.weight, None)):
+            # A small fp32 block: the four projections of x in one launch.
+            dt_raw, g_raw, Bq, Cq = f32_small_linears(x, dtp.weight, dtp.bias, gp.weight, gp.bias,
+                                                      bp.weight, None, cp.weight, None)
+            Bq, Cq = (m.view(b, t, D, self.d_state, 4) for m in (Bq, Cq))
+        else:
+            dt_raw, g_raw = _linear_pair(dtp, gp, x)
         if not recording and self._use_fused_bc(x):
             delta, s = ssm_front(dt_raw, g_raw, x)
             # Under autocast the projections' operands in its dtype, as F.linear casts them.
@@ -611,7 +642,8 @@ class QuaternionMamba2Block(nn.Module):
                     self.Lambda_imag, self.D, h0, width, self.d_state, 1e-6, self._gemm_dtype(x))
                 return (y, h) if return_state else y
             return self._ssm_forward_sliced(x, dt_raw, g_raw, width, h0, return_state)
-        Bq, Cq = _bc_pair(self.B_proj, self.C_proj, x, self.d_state)
+        if Bq is None:
+            Bq, Cq = _bc_pair(self.B_proj, self.C_proj, x, self.d_state)
         return ssm_forward_front_dl(dt_raw, g_raw, x, Bq, Cq, self.Lambda_alpha,
                                     self.Lambda_imag, self.D, eps=1e-6, h0=h0,
                                     return_state=return_state)

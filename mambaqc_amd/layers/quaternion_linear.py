@@ -10,6 +10,7 @@ torch F.linear (hipBLASLt on MI355X); the quaternion layout is a view:
 """
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -200,8 +201,8 @@ def _plain_call(*tensors) -> bool:
     """Plain dense tensors called eagerly: no tensor subclass (fake tensors), no dispatch
     mode, tracing, functorch transform or forward-mode AD in progress, all of which torch's
     own operators take part in and a direct launch does not."""
-    return (all(type(t) in (torch.Tensor, nn.Parameter) and t.layout == torch.strided and not t.is_neg()
-                for t in tensors)
+    return (all(type(t) in (torch.Tensor, nn.Parameter) and t.layout == torch.strided
+                and not t.is_neg() for t in tensors)
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None
@@ -217,6 +218,68 @@ def _f32_linear_eligible(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and not torch.is_autocast_enabled(x.device.type))
 
 
+# Small fp32 products of inference: torch's dispatch of one hipBLASLt fp32 GEMM takes 21 us of
+# host time whatever its size, mqc_gemm_f32_small about 8 for up to four. At this many FLOP and
+# this long a k the GPU is no slower with it (400 x 1024 x 256, 0.2 GFLOP: 9 us, hipBLASLt 10);
+# longer k or more work belongs to kernels that split k or fill the chip.
+F32_SMALL_MAX_FLOP = 6e8
+F32_SMALL_MAX_K = 2048
+
+
+def _f32_small_shape(M: int, N: int, K: int) -> bool:
+    return M > 0 and N > 0 and 0 < K <= F32_SMALL_MAX_K and 2.0 * M * N * K <= F32_SMALL_MAX_FLOP
+
+
+def _f32_small_launch(x: torch.Tensor, params, out) -> None:
+    """out_i = x w_i^T + b_i for x [M, K] with dense rows and (w_i [N_i, K] dense, b_i or None)
+    flat in params."""
+    M, K = x.shape
+    flat = []
+    for i, y in enumerate(out):
+        w, b = params[2 * i], params[2 * i + 1]
+        flat += (x.data_ptr(), x.stride(0), 1, w.data_ptr(), K, 1, 0 if b is None else b.data_ptr(),
+                 y.data_ptr(), M, w.shape[0], K)
+    nat.call("mqc_gemm_f32_small", x, (ctypes.c_int64 * len(flat))(*flat), len(out),
+             nat.stream_of(x))
+
+
+def f32_small_eligible(x: torch.Tensor, *params) -> bool:
+    """Whether F.linear(x, w, b) for every (w, b) in params (flat) runs as one launch of small
+    fp32 products: nothing recording autograd (a training step's backward from Python costs
+    more host time than the forward's launches save), plain tensors, dense rows."""
+    if x.dtype != torch.float32 or not x.is_cuda or x.dim() < 2:
+        return False
+    K = x.shape[-1]
+    rows = x.numel() // K if K else 0
+    grad = torch.is_grad_enabled()
+    if grad and x.requires_grad:
+        return False
+    columns = 0
+    for w, b in zip(params[0::2], params[1::2]):
+        if (w.dtype != torch.float32 or w.device != x.device or w.dim() != 2
+                or w.shape[1] != K or not w.is_contiguous() or (grad and w.requires_grad)):
+            return False
+        if b is not None and (b.dtype != torch.float32 or b.device != x.device or b.dim() != 1
+                              or not b.is_contiguous() or b.shape[0] != w.shape[0]
+                              or (grad and b.requires_grad)):
+            return False
+        columns += w.shape[0]
+    return (_f32_small_shape(rows, columns, K) and not torch.is_autocast_enabled(x.device.type)
+            and _plain_call(x, *params[0::2]))
+
+
+def f32_small_linears(x: torch.Tensor, *params):
+    """F.linear(x, w, b) for each of up to four (w, b) in params (flat; f32_small_eligible), in
+    one launch. Returns a tuple."""
+    x2 = x.detach().reshape(-1, x.shape[-1])
+    if x2.stride(1) != 1:
+        x2 = x2.contiguous()
+    out = [torch.empty(*x.shape[:-1], w.shape[0], device=x.device, dtype=torch.float32)
+           for w in params[0::2]]
+    _f32_small_launch(x2, params, out)
+    return tuple(out)
+
+
 def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """F.linear(x, weight) without bias, computed as column blocks of the
     output whose weight rows fit WIDE_LINEAR_CHUNK_BYTES, each written in place
@@ -227,9 +290,11 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     WIDE_LINEAR_MIN_ROWS rows; everything else takes F.linear. Under autocast
     the operands are cast to the autocast dtype, as F.linear's autocast rule
     does. Each output element is the same K-reduction as in one launch. fp32 products
-    that _f32_gemm_shape accepts run on the library's split GEMM instead, whatever their
-    weight's size.
+    that _f32_gemm_shape or _f32_small_shape accepts run on the library's own GEMMs
+    instead, whatever their weight's size.
     """
+    if f32_small_eligible(x, weight, None):
+        return f32_small_linears(x, weight, None)[0]
     if _f32_linear_eligible(x, weight):
         out = _F32MatmulT.apply(x.reshape(-1, x.shape[-1]), weight)
         return out.view(*x.shape[:-1], weight.shape[0])
@@ -366,6 +431,8 @@ class QuaternionLinear(nn.Module):
         if self.input_type == "quaternion":
             x = x.reshape(*x.shape[:-2], x.shape[-2] * 4)
         if self.output_type == "real":
+            if f32_small_eligible(x, self.weight, self.bias):
+                return f32_small_linears(x, self.weight, self.bias)[0]
             return F.linear(x, self.weight, self.bias)
         out = wide_linear(x, self.weight)
         out = out.view(*out.shape[:-1], self.out_features // 4, 4)
