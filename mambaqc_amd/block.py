@@ -225,13 +225,13 @@ def bc_slice_width(batch: int, seq_len: int, d_inner: int, d_state: int, elsize:
 
 def _unhooked(*layers: nn.Module) -> bool:
     """Plain nn.Linear layers without hooks, whose call is F.linear and nothing more."""
-    return all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks
+    return not nat.compiling() and all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks
                                              or m._backward_hooks or m._backward_pre_hooks)
                for m in layers)
 
 
 def _unhooked_quaternion(*layers) -> bool:
-    return all(type(m) is QuaternionLinear and not (m._forward_hooks or m._forward_pre_hooks
+    return not nat.compiling() and all(type(m) is QuaternionLinear and not (m._forward_hooks or m._forward_pre_hooks
                                                     or m._backward_hooks or m._backward_pre_hooks)
                for m in layers)
 

@@ -201,15 +201,18 @@ def _plain_call(*tensors) -> bool:
     """Plain dense tensors called eagerly: no tensor subclass (fake tensors), no dispatch
     mode, tracing, functorch transform or forward-mode AD in progress, all of which torch's
     own operators take part in and a direct launch does not."""
+    if torch.compiler.is_compiling():
+        return False
     return (all(type(t) in (torch.Tensor, nn.Parameter) and t.layout == torch.strided
                 and not t.is_neg() for t in tensors)
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0)
 
 
 def _f32_linear_eligible(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    if torch.compiler.is_compiling():
+        return False
     n, k = weight.shape
     rows = x.numel() // k if k else 0
     return (x.dtype == torch.float32 and weight.dtype == torch.float32
@@ -247,7 +250,8 @@ def f32_small_eligible(x: torch.Tensor, *params) -> bool:
     """Whether F.linear(x, w, b) for every (w, b) in params (flat) runs as one launch of small
     fp32 products: nothing recording autograd (a training step's backward from Python costs
     more host time than the forward's launches save), plain tensors, dense rows."""
-    if x.dtype != torch.float32 or not x.is_cuda or x.dim() < 2:
+    if (torch.compiler.is_compiling() or x.dtype != torch.float32 or not x.is_cuda
+            or x.dim() < 2):
         return False
     K = x.shape[-1]
     rows = x.numel() // K if K else 0
