@@ -30,6 +30,20 @@ int mqc_gemm_f32(const float* X, int64_t x_row, int64_t x_col, const float* W, i
  * bias (or 0), Y, M, N, K (pointers as integers; one of xm, xk and one of wn, wk is 1). */
 int mqc_gemm_f32_small(const int64_t* products, int64_t count, void* stream);
 
+/* mqc_qln_bwd with its parameter sums: dq, and dgamma [d] and dbeta [d, 4] in fp32. rows and d at least 1, d at most 4096; workspace of
+ * mqc_qln_bwd_sums_workspace_bytes(rows, d). */
+int64_t mqc_qln_bwd_sums_workspace_bytes(int64_t rows, int64_t d);
+int mqc_qln_bwd_sums(const void* q, const void* dout, const float* gamma, const float* mean,
+                     const float* rstd, void* dq, float* dgamma, float* dbeta, int64_t rows,
+                     int64_t d, float eps, int dtype, void* workspace, int64_t workspace_bytes,
+                     void* stream);
+
+/* out_i[c] = sum over r < rows of in_i[r * n_i + c] for up to three fp32 arrays (n_i 0: none),
+ * in a fixed order, in one launch. */
+int mqc_sum_rows(const float* in1, float* out1, int64_t n1, const float* in2, float* out2,
+                 int64_t n2, const float* in3, float* out3, int64_t n3, int64_t rows,
+                 void* stream);
+
 /* mqc_ssm_fused_bc_fwd for short sequences, seq_len from 1 to 128 (MQC_E_LIMIT above): same
  * operands, dtypes, shapes and refusals, in tiles of 64 or 128 tokens that hold whole
  * sequences of the batch, each group of 16 states in a workgroup of its own. d_state > 16

@@ -92,6 +92,9 @@ SIGNATURES_EXT = {
                      _vp],
     "mqc_ssm_fused_bc_short_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                    _i64, _i64, _i64, _i64, _f32, _int, _vp, _i64, _vp],
+    "mqc_qln_bwd_sums": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _int, _vp,
+                         _i64, _vp],
+    "mqc_sum_rows": [_vp, _vp, _i64] * 3 + [_i64, _vp],
     "mqc_gemm_f32_small": [_vp, _i64, _vp],
     "mqc_gemm_skinny4_nt": [_vp, _i64, _i64] + [_vp, _vp, _vp, _i64] * 4 + [_int, _vp],
     "mqc_step_in_proj_conv": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp,
@@ -103,6 +106,7 @@ SIGNATURES_EXT = {
                      _int, _vp],
 }
 SIGNATURES_EXT_I64 = {
+    "mqc_qln_bwd_sums_workspace_bytes": [_i64, _i64],
     "mqc_ssm_fused_bc_short_workspace_bytes": [_i64, _i64, _i64, _i64],
     "mqc_gemm_f32_workspace_bytes": [_i64, _i64, _i64],
 }

@@ -54,6 +54,18 @@ def _qln_backward(qc, g, mean, rstd, dout, eps):
     B, T, D, _ = qc.shape
     dout = nat.aligned16(dout.to(qc.dtype))
     dq = torch.empty_like(qc)
+    rows = B * T
+    nbytes = nat.load().mqc_qln_bwd_sums_workspace_bytes(rows, D) if rows and D else -1
+    if nbytes > 0:
+        # dgamma and dbeta summed inside (d_model up to 4096).
+        ws = torch.empty(nbytes, device=qc.device, dtype=torch.uint8)
+        dgamma = torch.empty(D, device=qc.device, dtype=torch.float32)
+        dbeta = torch.empty(D, 4, device=qc.device, dtype=torch.float32)
+        nat.call("mqc_qln_bwd_sums", qc, qc.data_ptr(), dout.data_ptr(), g.data_ptr(),
+                 mean.data_ptr(), rstd.data_ptr(), dq.data_ptr(), dgamma.data_ptr(),
+                 dbeta.data_ptr(), rows, D, float(eps), nat.dtype_code(qc), ws.data_ptr(), nbytes,
+                 nat.stream_of(qc))
+        return dq, dgamma, dbeta
     ne = torch.empty(B * T, D, device=qc.device, dtype=torch.float32)
     nat.call("mqc_qln_bwd", qc, qc.data_ptr(), dout.data_ptr(), g.data_ptr(),
              mean.data_ptr(), rstd.data_ptr(), dq.data_ptr(), ne.data_ptr(), B * T, D,

@@ -239,7 +239,16 @@ def ssm_fused_dl_backward(saved, gy, gh_last=None, eps: float = 1e-6,
                  d_s.data_ptr(), dB.data_ptr(), dC.data_ptr(), dla.data_ptr(), dli.data_ptr(),
                  dD.data_ptr(), nat.ptr(dh0), batch, T, d_inner, d_state, float(eps), code,
                  nat.stream_of(Bc))
-    return d_delta, d_s, dB, dC, dla.sum(0), dli.sum(0), dD.sum(0), dh0
+    if rows == 1:
+        return d_delta, d_s, dB, dC, dla[0], dli[0], dD[0], dh0
+    if rows == 0:
+        return d_delta, d_s, dB, dC, dla.sum(0), dli.sum(0), dD.sum(0), dh0
+    # The partials' sums over their rows, in one launch (three reductions of torch 28 us at 16 rows).
+    sums = [torch.empty(p.shape[1:], device=dev, dtype=torch.float32) for p in (dla, dli, dD)]
+    nat.call("mqc_sum_rows", dla, *(a for p, o in zip((dla, dli, dD), sums)
+                                    for a in (p.data_ptr(), o.data_ptr(), o.numel())),
+             rows, nat.stream_of(dla))
+    return d_delta, d_s, dB, dC, *sums, dh0
 
 
 class _SsmFusedDL(torch.autograd.Function):
