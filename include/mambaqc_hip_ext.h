@@ -44,6 +44,21 @@ int mqc_sum_rows(const float* in1, float* out1, int64_t n1, const float* in2, fl
                  int64_t n2, const float* in3, float* out3, int64_t n3, int64_t rows,
                  void* stream);
 
+/* mqc_cumprod_scan_fwd and mqc_ssm_q_fwd (from a zero state, without h_last) with the sequence
+ * in chunks of chunk_len steps walked side by side, for few lanes (batch x lanes, lanes =
+ * d_model x d_state for the SSM). chunk_len < seq_len; workspace (16-byte aligned) of
+ * mqc_q_chunked_workspace_bytes (ssm 1 for the SSM); batch x chunks at most 65535. */
+int64_t mqc_q_chunked_workspace_bytes(int64_t batch, int64_t seq_len, int64_t lanes,
+                                      int64_t chunk_len, int ssm);
+int mqc_cumprod_scan_chunked(const void* q, void* out, int64_t batch, int64_t seq_len,
+                             int64_t lanes, int64_t chunk_len, int dtype, void* workspace,
+                             int64_t workspace_bytes, void* stream);
+int mqc_ssm_q_fwd_chunked(const void* q, const void* B, const void* Sq, const void* C, const void* D,
+                          int64_t d_stride_b, int64_t d_stride_t, int64_t d_stride_d, void* y,
+                          int64_t batch, int64_t seq_len, int64_t d_model, int64_t d_state,
+                          int64_t chunk_len, int dtype, void* workspace, int64_t workspace_bytes,
+                          void* stream);
+
 /* mqc_ssm_fused_bc_fwd for short sequences, seq_len from 1 to 128 (MQC_E_LIMIT above): same
  * operands, dtypes, shapes and refusals, in tiles of 64 or 128 tokens that hold whole
  * sequences of the batch, each group of 16 states in a workgroup of its own. d_state > 16

@@ -95,6 +95,9 @@ SIGNATURES_EXT = {
     "mqc_qln_bwd_sums": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _int, _vp,
                          _i64, _vp],
     "mqc_sum_rows": [_vp, _vp, _i64] * 3 + [_i64, _vp],
+    "mqc_cumprod_scan_chunked": [_vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp],
+    "mqc_ssm_q_fwd_chunked": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64,
+                              _i64, _i64, _int, _vp, _i64, _vp],
     "mqc_gemm_f32_small": [_vp, _i64, _vp],
     "mqc_gemm_skinny4_nt": [_vp, _i64, _i64] + [_vp, _vp, _vp, _i64] * 4 + [_int, _vp],
     "mqc_step_in_proj_conv": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp,
@@ -107,6 +110,7 @@ SIGNATURES_EXT = {
 }
 SIGNATURES_EXT_I64 = {
     "mqc_qln_bwd_sums_workspace_bytes": [_i64, _i64],
+    "mqc_q_chunked_workspace_bytes": [_i64, _i64, _i64, _i64, _int],
     "mqc_ssm_fused_bc_short_workspace_bytes": [_i64, _i64, _i64, _i64],
     "mqc_gemm_f32_workspace_bytes": [_i64, _i64, _i64],
 }
@@ -188,6 +192,16 @@ def compiling() -> bool:
     registered torch.ops.mambaqc.* operators (traceable through their fake
     kernels) instead of ctypes."""
     return torch.compiler.is_compiling()
+
+
+def q_chunk_len(batch: int, seq_len: int, lanes: int, elsize: int) -> int:
+    """Steps per chunk of the time-chunked walks over a materialised q (csrc/q_chunk.hip): enough
+    chunks that batch x lanes x chunks x elsize is about 512 KiB, 8 to 64 of them, whole groups
+    of 8 steps and at least 16. Best of 16 to 512 steps in a sweep, SSM q form (T 4096 unless
+    noted): fp32 1024 lanes 64 steps, 4096 128, 8192 256, 24576 (T 2000) 256; bf16 4096 64, 8192
+    128, 24576 (T 2000) 128, 16000 (T 256) 16."""
+    n = min(64, max(8, (512 << 10) // max(1, batch * lanes * elsize)))
+    return max(16, -(-(-(-seq_len // n)) // 8) * 8)
 
 
 # The raw forms of torch.cuda.current_stream(device).cuda_stream and current_device(): a call's

@@ -14,6 +14,22 @@ import torch
 from .. import _native as nat
 
 
+# The time-chunked product (mqc_cumprod_scan_chunked) reads q twice, so it pays where the whole
+# walk is bound by its serial chain (us, whole / chunked): fp32 T 4096 1024 lanes 184 / 53, 4096
+# 190 / 141, but 8192 263 / 318; bf16 1024 435 / 38, 24576 (T 2000) 383 / 235, 16000 (T 256)
+# 33 / 23, 49152 (T 2000) 463 / 430.
+CHUNK_MAX_LANES = {4: 4096, 2: 24576}   # batch x lanes, by element size
+CHUNK_MIN_SEQ = {4: 512, 2: 128}
+
+
+def _chunk_len(B: int, T: int, lanes: int, el: int) -> int:
+    """Steps per chunk, 0 for the whole walk."""
+    if lanes < 1 or B * lanes > CHUNK_MAX_LANES[el] or T < CHUNK_MIN_SEQ[el]:
+        return 0
+    L = nat.q_chunk_len(B, T, lanes, el)
+    return L if L < T and B * -(-T // L) <= 65535 else 0
+
+
 def parallel_scan_quaternion(q_sequence: torch.Tensor) -> torch.Tensor:
     """q_sequence: [batch, seq_len, d_model, d_state, 4] -> cumulative products (new tensor)."""
     assert q_sequence.shape[-1] == 4
@@ -22,6 +38,13 @@ def parallel_scan_quaternion(q_sequence: torch.Tensor) -> torch.Tensor:
     q = nat.aligned16(q_sequence)
     B, T, D, S, _ = q.shape
     out = torch.empty_like(q)
+    L = _chunk_len(B, T, D * S, q.element_size())
+    if L:
+        nbytes = int(nat.load().mqc_q_chunked_workspace_bytes(B, T, D * S, L, 0))
+        ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
+        nat.call("mqc_cumprod_scan_chunked", q, q.data_ptr(), out.data_ptr(), B, T, D * S, L,
+                 nat.dtype_code(q), ws.data_ptr(), nbytes, nat.stream_of(q))
+        return out
     nat.call("mqc_cumprod_scan_fwd", q, q.data_ptr(), out.data_ptr(), B, T, D * S,
              nat.dtype_code(q), nat.stream_of(q))
     return out

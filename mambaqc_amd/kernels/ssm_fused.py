@@ -34,6 +34,22 @@ def _d_strides(D: torch.Tensor, dtype: torch.dtype):
     return D, tuple(D.stride())
 
 
+# The time-chunked q form (mqc_ssm_q_fwd_chunked) reads q and B twice, so it pays where the whole
+# walk is bound by its serial chain, 0.4 us a step (us, whole / chunked): fp32 T 4096 1024 lanes
+# 1661 / 84, 8192 1774 / 456, 24576 (T 2000) 843 / 646, but 49152 924 / 1367; bf16 8192 1709 / 251,
+# 49152 (T 2000) 868 / 697; T 150 3200 lanes 63 / 22.
+Q_CHUNK_MAX_BYTES = 96 << 10  # batch x lanes x element size
+Q_CHUNK_MIN_SEQ = 64
+
+
+def _q_chunk_len(batch: int, T: int, lanes: int, el: int) -> int:
+    """Steps per chunk of the q form, 0 for the whole walk."""
+    if lanes < 1 or batch * lanes * el > Q_CHUNK_MAX_BYTES or T < Q_CHUNK_MIN_SEQ:
+        return 0
+    L = nat.q_chunk_len(batch, T, lanes, el)
+    return L if L < T and batch * -(-T // L) <= 65535 else 0
+
+
 def _launch_q(q, B, S, C, D, h0, batch, T, d_model, d_state, name, want_state):
     dtype = q.dtype
     for t in (B, S, C):
@@ -48,6 +64,16 @@ def _launch_q(q, B, S, C, D, h0, batch, T, d_model, d_state, name, want_state):
         if h0.dtype != dtype:
             raise TypeError(f"{name}: dtype mismatch {dtype} vs {h0.dtype}")
         h0 = nat.aligned16(h0)
+    L = 0
+    if h0 is None and not want_state and d_state <= 256:
+        L = _q_chunk_len(batch, T, d_model * d_state, q.element_size())
+    if L:
+        nbytes = int(nat.load().mqc_q_chunked_workspace_bytes(batch, T, d_model * d_state, L, 1))
+        ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
+        nat.call("mqc_ssm_q_fwd_chunked", q, q.data_ptr(), B.data_ptr(), S.data_ptr(),
+                 C.data_ptr(), Dt.data_ptr(), sb, st, sd, y.data_ptr(), batch, T, d_model,
+                 d_state, L, nat.dtype_code(q), ws.data_ptr(), nbytes, nat.stream_of(q))
+        return y, h_last
     nat.call("mqc_ssm_q_fwd", q, q.data_ptr(), B.data_ptr(), S.data_ptr(), C.data_ptr(),
              Dt.data_ptr(), sb, st, sd, nat.ptr(h0), y.data_ptr(), nat.ptr(h_last),
              batch, T, d_model, d_state, nat.dtype_code(q), nat.stream_of(q))
