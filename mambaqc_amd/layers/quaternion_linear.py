@@ -192,8 +192,9 @@ class _F32MatmulT(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gy):
         x, w = ctx.saved_tensors
-        gx = _F32MatmulT.apply(gy, w.t()) if ctx.needs_input_grad[0] else None
-        gw = _F32MatmulT.apply(gy.t(), x.t()) if ctx.needs_input_grad[1] else None
+        mm = _F32MatmulT.apply if torch.is_grad_enabled() else _f32_mm_t
+        gx = mm(gy, w.t()) if ctx.needs_input_grad[0] else None
+        gw = mm(gy.t(), x.t()) if ctx.needs_input_grad[1] else None
         return gx, gw
 
 
