@@ -17,8 +17,8 @@
 //   - Row scale: 2^(14 - exponent of the row's largest |a|), so hi never overflows; taken
 //     back in the epilogue with ldexp. amax holds each row's largest |a| (as fp32 bits, the
 //     maximum taken on the bits, so that an inf or a NaN is the largest).
-//   - Rows with an inf or a NaN: their amax says so, and the epilogue computes those rows'
-//     outputs from the fp32 operands with a plain fp32 loop.
+//   - Rows with a NaN or an inf: their amax says so; a NaN row's outputs are NaN, and those of a
+//     row with an inf are computed in the epilogue from the fp32 operands with a plain fp32 loop.
 //   - Layout of the pieces: per row and 32 columns of k, 32 hi pieces and then 32 lo pieces
 //     (128 bytes: one K step of mfma_tile.hpp's loop), columns past K zero.
 //   - Blocks: an operand is split a block at a time (kBlockElems, 64 MiB of pieces), and each
@@ -294,15 +294,22 @@ __global__ __launch_bounds__(Cfg::kThreads) void gemm_f32_kernel(GemmF32Args a) 
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = __builtin_amdgcn_ldexpf(acc[nb][mb][i], -(xe + we[i]));
       if (bad_w || not_finite(xm1)) {
-        // A row with an inf or a NaN: the plain fp32 sum of this share of k.
+        // A row with a NaN has nothing but NaNs in its outputs; one with an inf takes the plain
+        // fp32 sum of this share of k.
         const int k1 = s_hi * kChunk < a.K ? s_hi * kChunk : a.K;
 #pragma unroll 1
         for (int i = 0; i < 4; ++i) {
           if (nn + i >= a.N) break;
+          const float wmax = i == 0 ? wm4[0] : i == 1 ? wm4[1] : i == 2 ? wm4[2] : wm4[3];
+          if (!(not_finite(xm1) || not_finite(wmax))) continue;
           float sum = 0.f;
+          if (xm1 != xm1 || wmax != wmax) {
+            sum = __uint_as_float(0x7fc00000u);
+          } else {
 #pragma unroll 1
-          for (int k = s_lo * kChunk; k < k1; ++k)
-            sum = fmaf(a.X[m * a.xm + k * a.xk], a.W[(nn + i) * a.wn + k * a.wk], sum);
+            for (int k = s_lo * kChunk; k < k1; ++k)
+              sum = fmaf(a.X[m * a.xm + k * a.xk], a.W[(nn + i) * a.wn + k * a.wk], sum);
+          }
           v[0] = i == 0 ? sum : v[0];
           v[1] = i == 1 ? sum : v[1];
           v[2] = i == 2 ? sum : v[2];
