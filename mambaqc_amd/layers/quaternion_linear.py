@@ -160,13 +160,10 @@ def _unit_rows(t: torch.Tensor) -> torch.Tensor:
     return t if ok else t.contiguous()
 
 
-def _f32_mm_t(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x w^T in fp32, x [M, K] and w [N, K] (or transposed views): on mqc_gemm_f32 where it
-    is faster, else torch's."""
+def _f32_launch(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T on mqc_gemm_f32."""
     M, K = x.shape
     N = w.shape[0]
-    if not _f32_gemm_shape(M, N, K):
-        return torch.mm(x, w.t())
     x, w = _unit_rows(x), _unit_rows(w)
     lib = nat.load()
     nbytes = int(lib.mqc_gemm_f32_workspace_bytes(M, N, K))
@@ -180,32 +177,57 @@ def _f32_mm_t(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return y
 
 
+def _f32_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.is_cuda
+            and w.device == x.device)
+
+
+def _f32_eligible(x: torch.Tensor, w: torch.Tensor, rows: int) -> bool:
+    """Whether x w^T, x of `rows` rows, runs on mqc_gemm_f32."""
+    n, k = w.shape
+    return (_f32_operands(x, w) and _f32_gemm_shape(rows, n, k) and _plain_call(x, w)
+            and not torch.is_autocast_enabled(x.device.type))
+
+
+def _f32_mm_t(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T in fp32, x [M, K] and w [N, K] (or transposed views): on mqc_gemm_f32 where it
+    is faster and may be launched directly, else torch's."""
+    if not _f32_eligible(x, w, x.shape[0]):
+        return torch.mm(x, w.t())
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return _F32MatmulT.apply(x, w)
+    return _f32_launch(x, w)
+
+
 class _F32MatmulT(torch.autograd.Function):
     """x w^T in fp32. Its gradients are products of the same kind (gy w and gy^T x), made by
-    the same function, so gradients of gradients exist as for torch's."""
+    the same function, so gradients of gradients exist as for torch's. The incoming gradient
+    and the saved operands are looked at again there: a gradient may be batched
+    (is_grads_batched), carry a forward-mode tangent or a lazy negation, or arrive under
+    autocast, where the forward's operands did not."""
 
     @staticmethod
     def forward(ctx, x, w):
         ctx.save_for_backward(x, w)
-        return _f32_mm_t(x, w)
+        return _f32_launch(x, w)
 
     @staticmethod
     def backward(ctx, gy):
         x, w = ctx.saved_tensors
-        mm = _F32MatmulT.apply if torch.is_grad_enabled() else _f32_mm_t
-        gx = mm(gy, w.t()) if ctx.needs_input_grad[0] else None
-        gw = mm(gy.t(), x.t()) if ctx.needs_input_grad[1] else None
+        gx = _f32_mm_t(gy, w.t()) if ctx.needs_input_grad[0] else None
+        gw = _f32_mm_t(gy.t(), x.t()) if ctx.needs_input_grad[1] else None
         return gx, gw
 
 
 def _plain_call(*tensors) -> bool:
-    """Plain dense tensors called eagerly: no tensor subclass (fake tensors), no dispatch
-    mode, tracing, functorch transform or forward-mode AD in progress, all of which torch's
-    own operators take part in and a direct launch does not."""
+    """Plain dense tensors called eagerly: no tensor subclass (fake tensors), no wrapper
+    without storage (the batched gradients of autograd.grad, which show in no other way), no
+    dispatch mode, tracing, functorch transform or forward-mode AD in progress, all of which
+    torch's own operators take part in and a direct launch does not."""
     if torch.compiler.is_compiling():
         return False
     return (all(type(t) in (torch.Tensor, nn.Parameter) and t.layout == torch.strided
-                and not t.is_neg() for t in tensors)
+                and torch._C._has_storage(t) and not t.is_neg() for t in tensors)
             and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0)
@@ -214,12 +236,8 @@ def _plain_call(*tensors) -> bool:
 def _f32_linear_eligible(x: torch.Tensor, weight: torch.Tensor) -> bool:
     if torch.compiler.is_compiling():
         return False
-    n, k = weight.shape
-    rows = x.numel() // k if k else 0
-    return (x.dtype == torch.float32 and weight.dtype == torch.float32
-            and x.is_cuda and weight.device == x.device and x.shape[-1] == k
-            and _f32_gemm_shape(rows, n, k) and _plain_call(x, weight)
-            and not torch.is_autocast_enabled(x.device.type))
+    k = weight.shape[1]
+    return x.shape[-1] == k and _f32_eligible(x, weight, x.numel() // k if k else 0)
 
 
 # Small fp32 products of inference: torch's dispatch of one hipBLASLt fp32 GEMM takes 21 us of

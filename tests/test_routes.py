@@ -1,0 +1,109 @@
+"""Which calls take the library's fp32 products and which stay with torch's operators, on the
+CPU: the launch is emulated from the pointers that the host code hands over."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+from torch.autograd import forward_ad as fa
+
+import mambaqc_amd.layers.quaternion_linear as ql
+from mambaqc_amd import _native as nat
+
+
+def _at(ptr, r, c, rs, cs):
+    """The fp32 matrix [r, c] at ptr with strides in elements, as the kernel reads it."""
+    n = (r - 1) * rs + (c - 1) * cs + 1
+    flat = np.ctypeslib.as_array((ctypes.c_float * n).from_address(ptr))
+    return np.lib.stride_tricks.as_strided(flat, (r, c), (4 * rs, 4 * cs))
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """Every fp32 product on the emulated kernel; the list of the shapes launched."""
+    seen = []
+
+    def call(name, _, xp, xr, xc, wp, wr, wc, yp, ldy, M, N, K, *rest):
+        assert name == "mqc_gemm_f32"
+        seen.append((M, N, K))
+        _at(yp, M, N, ldy, 1)[:] = _at(xp, M, K, xr, xc) @ _at(wp, N, K, wr, wc).T
+
+    monkeypatch.setattr(nat, "call", call)
+    monkeypatch.setattr(nat, "stream_of", lambda t: 0)
+    monkeypatch.setattr(ql, "_f32_gemm_shape", lambda M, N, K: True)
+    monkeypatch.setattr(ql, "_f32_operands", lambda x, w: x.dtype == w.dtype == torch.float32,
+                        raising=False)
+    return seen
+
+
+def _operands():
+    g = torch.Generator().manual_seed(5)
+    r = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    return r(6, 5).requires_grad_(), r(7, 5).requires_grad_(), r(6, 7), r(6, 7)
+
+
+def _close(got, ref):
+    for a, b in zip(got, ref):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
+def test_gradients_on_the_kernel(launches):
+    x, w, gy, _ = _operands()
+    got = torch.autograd.grad(ql._F32MatmulT.apply(x, w), (x, w), gy)
+    assert launches == [(6, 7, 5), (6, 5, 7), (7, 5, 6)]
+    _close(got, torch.autograd.grad(F.linear(x, w), (x, w), gy))
+
+
+def test_forward_mode_tangent_of_the_gradient(launches):
+    """The product made outside a dual level, its gradient taken inside one."""
+    x, w, gy, t = _operands()
+
+    def tangents(y):
+        with fa.dual_level():
+            g = torch.autograd.grad(y, (x, w), fa.make_dual(gy, t))
+            return [fa.unpack_dual(a).tangent for a in g]
+
+    ref = tangents(F.linear(x, w))
+    got = tangents(ql._F32MatmulT.apply(x, w))
+    assert all(a is not None for a in got)
+    _close(got, ref)
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_batched_gradients(launches, create_graph):
+    x, w, _, _ = _operands()
+    gy = torch.randn(3, 6, 7, requires_grad=create_graph)
+    grads = lambda y: torch.autograd.grad(  # noqa: E731
+        y, (x, w), gy, is_grads_batched=True, create_graph=create_graph)
+    _close(grads(ql._F32MatmulT.apply(x, w)), grads(F.linear(x, w)))
+
+
+def test_lazily_negated_gradient(launches):
+    x, w, gy, _ = _operands()
+    neg = torch._neg_view(gy)  # (as the imaginary part of a conjugate is)
+
+    class Hand(torch.autograd.Function):  # (passes a gradient on as it is)
+        @staticmethod
+        def forward(ctx, y):
+            return y.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return neg
+
+    got, ref = (torch.autograd.grad(Hand.apply(f(x, w)).sum(), (x, w))
+                for f in (ql._F32MatmulT.apply, F.linear))
+    _close(got, ref)
+
+
+def test_gradient_under_autocast(launches):
+    """F.linear's gradients are autocast where the backward itself runs under autocast."""
+    x, w, gy, _ = _operands()
+
+    def grads(y):
+        with torch.autocast("cpu", dtype=torch.bfloat16):
+            return torch.autograd.grad(y, (x, w), gy)
+
+    got, ref = grads(ql._F32MatmulT.apply(x, w)), grads(F.linear(x, w))
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
