@@ -24,7 +24,7 @@ CHUNK_MIN_SEQ = {4: 512, 2: 128}
 
 def _chunk_len(B: int, T: int, lanes: int, el: int) -> int:
     """Steps per chunk, 0 for the whole walk."""
-    if lanes < 1 or B * lanes > CHUNK_MAX_LANES[el] or T < CHUNK_MIN_SEQ[el]:
+    if B < 1 or lanes < 1 or B * lanes > CHUNK_MAX_LANES[el] or T < CHUNK_MIN_SEQ[el]:
         return 0
     L = nat.q_chunk_len(B, T, lanes, el)
     return L if L < T and B * -(-T // L) <= 65535 else 0

@@ -44,7 +44,8 @@ Q_CHUNK_MIN_SEQ = 64
 
 def _q_chunk_len(batch: int, T: int, lanes: int, el: int) -> int:
     """Steps per chunk of the q form, 0 for the whole walk."""
-    if lanes < 1 or batch * lanes * el > Q_CHUNK_MAX_BYTES or T < Q_CHUNK_MIN_SEQ:
+    if (batch < 1 or lanes < 1 or batch * lanes * el > Q_CHUNK_MAX_BYTES
+            or T < Q_CHUNK_MIN_SEQ):
         return 0
     L = nat.q_chunk_len(batch, T, lanes, el)
     return L if L < T and batch * -(-T // L) <= 65535 else 0

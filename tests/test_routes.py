@@ -1,5 +1,6 @@
-"""Which calls take the library's fp32 products and which stay with torch's operators, on the
-CPU: the launch is emulated from the pointers that the host code hands over."""
+"""Which calls take which of the library's paths and which stay with torch's operators, on the
+CPU: an fp32 product's launch is emulated from the pointers that the host code hands over, and
+calls that end in the library's host code run it."""
 import ctypes
 
 import numpy as np
@@ -10,6 +11,7 @@ from torch.autograd import forward_ad as fa
 
 import mambaqc_amd.layers.quaternion_linear as ql
 from mambaqc_amd import _native as nat
+from mambaqc_amd import kernels as K
 
 
 def _at(ptr, r, c, rs, cs):
@@ -107,3 +109,26 @@ def test_gradient_under_autocast(launches):
 
     got, ref = grads(ql._F32MatmulT.apply(x, w)), grads(F.linear(x, w))
     assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+@pytest.fixture
+def host_code(monkeypatch):
+    """Calls reach the built library's host code, with CPU tensors."""
+    def call(name, _, *args):
+        nat.check(getattr(nat.load(), name)(*args), name)
+
+    monkeypatch.setattr(nat, "call", call)
+    monkeypatch.setattr(nat, "stream_of", lambda t: 0)
+    monkeypatch.setattr(nat, "require_device", lambda *a: None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(0, 600, 4, 16), (0, 64, 1, 1), (2, 600, 0, 16), (1, 600, 4, 0)])
+def test_empty_scans(host_code, dtype, shape):
+    """No batch, no channel, no state: nothing to launch, an empty result."""
+    b, t, d, s = shape
+    q = torch.empty(b, t, d, s, 4, dtype=dtype)
+    assert K.parallel_scan_quaternion(q).shape == q.shape
+    if s:  # (without states y is a sum of none, which the kernel writes)
+        S, D = torch.empty(b, t, d, 4, dtype=dtype), torch.empty(b, t, d, dtype=dtype)
+        assert K.ssm_forward_fused(q, q, S, q, D).shape == S.shape
