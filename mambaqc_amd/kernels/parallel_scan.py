@@ -35,6 +35,7 @@ def parallel_scan_quaternion(q_sequence: torch.Tensor) -> torch.Tensor:
     assert q_sequence.shape[-1] == 4
     assert q_sequence.ndim == 5
     nat.require_device("parallel_scan_quaternion", q_sequence)
+    code = nat.dtype_code(q_sequence)
     q = nat.aligned16(q_sequence)
     B, T, D, S, _ = q.shape
     out = torch.empty_like(q)
@@ -43,8 +44,8 @@ def parallel_scan_quaternion(q_sequence: torch.Tensor) -> torch.Tensor:
         nbytes = int(nat.load().mqc_q_chunked_workspace_bytes(B, T, D * S, L, 0))
         ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
         nat.call("mqc_cumprod_scan_chunked", q, q.data_ptr(), out.data_ptr(), B, T, D * S, L,
-                 nat.dtype_code(q), ws.data_ptr(), nbytes, nat.stream_of(q))
+                 code, ws.data_ptr(), nbytes, nat.stream_of(q))
         return out
     nat.call("mqc_cumprod_scan_fwd", q, q.data_ptr(), out.data_ptr(), B, T, D * S,
-             nat.dtype_code(q), nat.stream_of(q))
+             code, nat.stream_of(q))
     return out

@@ -132,3 +132,13 @@ def test_empty_scans(host_code, dtype, shape):
     if s:  # (without states y is a sum of none, which the kernel writes)
         S, D = torch.empty(b, t, d, 4, dtype=dtype), torch.empty(b, t, d, dtype=dtype)
         assert K.ssm_forward_fused(q, q, S, q, D).shape == S.shape
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.int32])
+def test_scans_name_a_dtype_they_do_not_take(host_code, dtype):
+    q = torch.zeros(1, 600, 2, 4, 4, dtype=dtype)
+    with pytest.raises(TypeError, match="unsupported dtype"):
+        K.parallel_scan_quaternion(q)
+    with pytest.raises(TypeError, match="unsupported dtype"):
+        K.ssm_forward_fused(q, q, torch.zeros(1, 600, 2, 4, dtype=dtype), q,
+                            torch.zeros(1, 600, 2, dtype=dtype))
