@@ -471,19 +471,23 @@ class QuaternionMamba2Block(nn.Module):
         state = (conv_tail, h): conv_tail [batch, d_conv - 1, d_inner] holds the
         last d_conv - 1 conv inputs, h [batch, d_inner, d_state, 4] the SSM
         state, in fp32 whatever the model dtype (the precision the walk
-        carries it in). None starts from zeros, where the result equals forward(x).
+        carries it in). None starts from zeros, where the result equals forward(x); so does
+        an h of None for the SSM alone.
         Feeding a sequence in pieces gives the same outputs as feeding it whole
         (up to rounding), which is what recurrent decoding relies on.
         """
         b, t, _ = x.shape
         if t == 1 and self._step_fused_ok(x):
             # One token: the decode step, on copies of the state.
+            tail, h = (None, None) if state is None else state
             if state is None:
                 tail = x.new_zeros(b, self.d_conv - 1, self.d_inner)
+            else:
+                tail = tail.to(x.dtype).clone(memory_format=torch.contiguous_format)
+            if h is None:
                 h = x.new_zeros(b, self.d_inner, self.d_state, 4, dtype=torch.float32)
             else:
-                tail = state[0].to(x.dtype).clone(memory_format=torch.contiguous_format)
-                h = state[1].to(torch.float32).clone(memory_format=torch.contiguous_format)
+                h = h.to(torch.float32).clone(memory_format=torch.contiguous_format)
             if self._step_state_ok(x, tail, h):
                 return self._step_fused(x, tail, h), (tail, h)
         xz = _linear(self.in_proj, x)

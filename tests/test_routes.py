@@ -11,6 +11,7 @@ from torch.autograd import forward_ad as fa
 
 import mambaqc_amd.layers.quaternion_linear as ql
 from mambaqc_amd import _native as nat
+from mambaqc_amd import block
 from mambaqc_amd import kernels as K
 
 
@@ -142,3 +143,36 @@ def test_scans_name_a_dtype_they_do_not_take(host_code, dtype):
     with pytest.raises(TypeError, match="unsupported dtype"):
         K.ssm_forward_fused(q, q, torch.zeros(1, 600, 2, 4, dtype=dtype), q,
                             torch.zeros(1, 600, 2, dtype=dtype))
+
+
+class Taken(Exception):
+    pass
+
+
+@pytest.fixture
+def one_token(monkeypatch):
+    """A bf16 block whose one-token call says which way it went."""
+    blk = block.QuaternionMamba2Block(64, d_state=4).bfloat16().eval()
+
+    def step(x, tail, h):
+        raise Taken("step", tail, h)
+
+    def separate(x, h0=None, return_state=False):
+        raise Taken("separate", h0)
+
+    monkeypatch.setattr(blk, "_step_fused_ok", lambda x: True)
+    monkeypatch.setattr(blk, "_step_fused", step)
+    monkeypatch.setattr(blk, "_ssm_forward", separate)
+    monkeypatch.setattr(block, "causal_conv1d_silu", lambda x, w, b: x)
+    return blk, torch.zeros(2, 1, 64, dtype=torch.bfloat16)
+
+
+def test_one_token_from_a_conv_tail_alone(one_token):
+    """A state without an SSM part starts the SSM from zeros."""
+    blk, x = one_token
+    tail = torch.randn(2, 3, 128)
+    with torch.no_grad(), pytest.raises(Taken) as e:
+        blk.forward_with_state(x, (tail, None))
+    way, t, h = e.value.args
+    assert way == "step" and torch.equal(t, tail.bfloat16())
+    assert h.shape == (2, 128, 4, 4) and h.dtype == torch.float32 and not h.any()
