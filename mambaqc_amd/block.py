@@ -477,8 +477,9 @@ class QuaternionMamba2Block(nn.Module):
         (up to rounding), which is what recurrent decoding relies on.
         """
         b, t, _ = x.shape
-        if t == 1 and self._step_fused_ok(x):
-            # One token: the decode step, on copies of the state.
+        if t == 1 and not self.fuse_bc and not self.bc_slice_d and self._step_fused_ok(x):
+            # One token: the decode step, on copies of the state (a forced way of the B/C
+            # projections is kept, and a refused one still refused).
             tail, h = (None, None) if state is None else state
             if state is None:
                 tail = x.new_zeros(b, self.d_conv - 1, self.d_inner)

@@ -176,3 +176,16 @@ def test_one_token_from_a_conv_tail_alone(one_token):
     way, t, h = e.value.args
     assert way == "step" and torch.equal(t, tail.bfloat16())
     assert h.shape == (2, 128, 4, 4) and h.dtype == torch.float32 and not h.any()
+
+
+@pytest.mark.parametrize("attr,value,way", [
+    ("fuse_bc", None, "step"), ("fuse_bc", False, "step"), ("fuse_bc", True, "separate"),
+    ("bc_slice_d", 0, "step"), ("bc_slice_d", 16, "separate"), ("bc_slice_d", -1, "separate")])
+def test_one_token_keeps_a_forced_way(one_token, attr, value, way):
+    """What a caller forces for the B/C projections holds for one token too (and a negative
+    slice width goes where it is refused)."""
+    blk, x = one_token
+    setattr(blk, attr, value)
+    with torch.no_grad(), pytest.raises(Taken) as e:
+        blk.forward_with_state(x)
+    assert e.value.args[0] == way
