@@ -35,6 +35,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _module
 
 from . import _native as nat
 from .kernels.quaternion_norm import QuaternionLayerNorm
@@ -223,17 +224,15 @@ def bc_slice_width(batch: int, seq_len: int, d_inner: int, d_state: int, elsize:
     return max(1, min(d_inner, budget // max(per_d, 1)))
 
 
-def _unhooked(*layers: nn.Module) -> bool:
-    """Plain nn.Linear layers without hooks, whose call is F.linear and nothing more."""
-    return not nat.compiling() and all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks
-                                             or m._backward_hooks or m._backward_pre_hooks)
-               for m in layers)
-
-
-def _unhooked_quaternion(*layers) -> bool:
-    return not nat.compiling() and all(type(m) is QuaternionLinear and not (m._forward_hooks or m._forward_pre_hooks
-                                                    or m._backward_hooks or m._backward_pre_hooks)
-               for m in layers)
+def _bare(kind: type, *layers: nn.Module) -> bool:
+    """Layers of exactly `kind` whose call is their class's forward and nothing more: no hooks of
+    their own or global ones, no replaced or compiled forward, and not while tracing."""
+    if (nat.compiling() or _module._global_forward_hooks or _module._global_forward_pre_hooks
+            or _module._global_backward_hooks or _module._global_backward_pre_hooks):
+        return False
+    return all(type(m) is kind and "forward" not in m.__dict__ and m._compiled_call_impl is None
+               and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                        or m._backward_pre_hooks) for m in layers)
 
 
 def _linear(layer: nn.Linear, x: torch.Tensor) -> torch.Tensor:
@@ -241,7 +240,7 @@ def _linear(layer: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     small fp32 ones."""
     if skinny_eligible(x, layer.weight, layer.bias):
         return skinny_linear(x, layer.weight, layer.bias)
-    if _unhooked(layer) and f32_small_eligible(x, layer.weight, layer.bias):
+    if _bare(nn.Linear, layer) and f32_small_eligible(x, layer.weight, layer.bias):
         return f32_small_linears(x, layer.weight, layer.bias)[0]
     return layer(x)
 
@@ -250,7 +249,7 @@ def _linear_pair(a: nn.Linear, b: nn.Linear, x: torch.Tensor):
     """(a(x), b(x)), in one skinny launch for decode-sized inputs."""
     if skinny_eligible(x, a.weight, a.bias, b.weight, b.bias):
         return skinny_linear(x, a.weight, a.bias, b.weight, b.bias)
-    if _unhooked(a, b) and f32_small_eligible(x, a.weight, a.bias, b.weight, b.bias):
+    if _bare(nn.Linear, a, b) and f32_small_eligible(x, a.weight, a.bias, b.weight, b.bias):
         return f32_small_linears(x, a.weight, a.bias, b.weight, b.bias)
     return a(x), b(x)
 
@@ -620,7 +619,7 @@ class QuaternionMamba2Block(nn.Module):
         dtp, gp, bp, cp = self.dt_proj, self.gate_proj, self.B_proj, self.C_proj
         Bq = Cq = None
         if (not recording and not width and bp.bias is None and cp.bias is None
-                and _unhooked(dtp, gp) and _unhooked_quaternion(bp, cp)
+                and _bare(nn.Linear, dtp, gp) and _bare(QuaternionLinear, bp, cp)
                 and f32_small_eligible(x, dtp.weight, dtp.bias, gp.weight, gp.bias,
                                        bp.weight, None, cp.weight, None)):
             # A small fp32 block: the four projections of x in one launch.

@@ -16,6 +16,7 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from .. import _native as nat
 
@@ -219,12 +220,19 @@ class _F32MatmulT(torch.autograd.Function):
         return gx, gw
 
 
+def _function_modes() -> bool:
+    """Whether a TorchFunctionMode sees torch's calls, other than a default device's, which
+    leaves products alone."""
+    return torch._C._len_torch_function_stack() > 0 and not all(
+        type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+
+
 def _plain_call(*tensors) -> bool:
     """Plain dense tensors called eagerly: no tensor subclass (fake tensors), no wrapper
     without storage (the batched gradients of autograd.grad, which show in no other way), no
-    dispatch mode, tracing, functorch transform or forward-mode AD in progress, all of which
-    torch's own operators take part in and a direct launch does not."""
-    if torch.compiler.is_compiling():
+    dispatch or function mode, tracing, functorch transform or forward-mode AD in progress, all
+    of which torch's own operators take part in and a direct launch does not."""
+    if torch.compiler.is_compiling() or _function_modes():
         return False
     return (all(type(t) in (torch.Tensor, nn.Parameter) and t.layout == torch.strided
                 and torch._C._has_storage(t) and not t.is_neg() for t in tensors)
@@ -288,7 +296,7 @@ def f32_small_eligible(x: torch.Tensor, *params) -> bool:
             return False
         columns += w.shape[0]
     return (_f32_small_shape(rows, columns, K) and not torch.is_autocast_enabled(x.device.type)
-            and _plain_call(x, *params[0::2]))
+            and _plain_call(x, *(p for p in params if p is not None)))
 
 
 def f32_small_linears(x: torch.Tensor, *params):

@@ -8,6 +8,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad as fa
+from torch.overrides import TorchFunctionMode
 
 import mambaqc_amd.layers.quaternion_linear as ql
 from mambaqc_amd import _native as nat
@@ -189,3 +190,56 @@ def test_one_token_keeps_a_forced_way(one_token, attr, value, way):
     with torch.no_grad(), pytest.raises(Taken) as e:
         blk.forward_with_state(x)
     assert e.value.args[0] == way
+
+
+class Count(TorchFunctionMode):
+    seen = 0
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        if func is F.linear:
+            self.seen += 1
+        return func(*args, **(kwargs or {}))
+
+
+def _way(monkeypatch):
+    """Whether block._linear took the library's product for a plain fp32 nn.Linear layer."""
+    taken = []
+    monkeypatch.setattr(block, "f32_small_eligible", lambda *a: True)
+    monkeypatch.setattr(block, "f32_small_linears", lambda x, w, b: taken.append(1) or [x @ w.t()])
+    return taken
+
+
+def test_bare_layers_only(monkeypatch):
+    """Global and own hooks run, and a replaced or compiled forward is called."""
+    taken, x = _way(monkeypatch), torch.randn(3, 8)
+    layer = torch.nn.Linear(8, 4, bias=False)
+    block._linear(layer, x)
+    assert taken == [1]
+    seen = []
+    register = torch.nn.modules.module
+    for hook in (register.register_module_forward_hook, register.register_module_forward_pre_hook,
+                 layer.register_forward_hook, layer.register_forward_pre_hook):
+        h = hook(lambda *a: seen.append(hook))
+        block._linear(layer, x)
+        h.remove()
+        assert seen[-1] is hook
+    layer.forward = lambda x: seen.append("own") or x
+    assert block._linear(layer, x) is x and seen[-1] == "own"
+    del layer.forward
+    layer._compiled_call_impl = lambda x: seen.append("compiled") or x
+    assert block._linear(layer, x) is x and seen[-1] == "compiled"
+    layer._compiled_call_impl = None
+    assert taken == [1]
+    block._linear(layer, x)
+    assert taken == [1, 1]
+
+
+def test_function_modes_see_the_product():
+    x, w = torch.randn(3, 8), torch.randn(4, 8)
+    assert ql._plain_call(x, w)
+    with torch.device("cpu"):
+        assert ql._plain_call(x, w)
+    with Count() as mode:
+        assert not ql._plain_call(x, w)
+        ql.wide_linear(x, w)
+    assert mode.seen == 1
