@@ -212,9 +212,12 @@ _raw_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def stream_of(t: torch.Tensor) -> int:
-    if _raw_stream is None:
+    """The current stream of t's device; raises for a tensor that is on none (the raw call would
+    answer with some device's stream, and a launch read host addresses)."""
+    idx = t.get_device()
+    if idx < 0 or _raw_stream is None:
         return torch.cuda.current_stream(t.device).cuda_stream
-    return _raw_stream(t.get_device())
+    return _raw_stream(idx)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -267,11 +270,14 @@ _fns: dict = {}
 def call(name: str, device_tensor: torch.Tensor, *args) -> None:
     """Call entry point `name` with the tensor's device current (the library
     launches on the device that is current; the stream argument must belong to
-    it). The device switch is skipped when it is current already."""
+    it). The device switch is skipped when it is current already. Raises for a
+    tensor on no device."""
+    idx = device_tensor.get_device()
+    if idx < 0:
+        raise RuntimeError(f"{name}: expected a tensor on a ROCm device, got {device_tensor.device}")
     fn = _fns.get(name)
     if fn is None:
         fn = _fns.setdefault(name, getattr(load(), name))
-    idx = device_tensor.get_device()
     if idx == (_raw_device() if _raw_device is not None else torch.cuda.current_device()):
         status = fn(*args)
     else:

@@ -10,6 +10,7 @@ import torch.nn.functional as F
 from torch.autograd import forward_ad as fa
 from torch.overrides import TorchFunctionMode
 
+import mambaqc_amd.ops  # noqa: F401
 import mambaqc_amd.layers.quaternion_linear as ql
 from mambaqc_amd import _native as nat
 from mambaqc_amd import block
@@ -243,3 +244,22 @@ def test_function_modes_see_the_product():
         assert not ql._plain_call(x, w)
         ql.wide_linear(x, w)
     assert mode.seen == 1
+
+
+def test_host_tensors_never_reach_a_launch(monkeypatch):
+    """On a machine with a GPU the raw stream and device calls answer for any index, -1 too; the
+    operators without a device check of their own stop at the stream of a host tensor."""
+    ran = []
+    monkeypatch.setattr(nat, "_raw_stream", lambda i: 0)
+    monkeypatch.setattr(nat, "_raw_device", lambda: -1)
+    monkeypatch.setattr(nat, "_fns", dict.fromkeys([*nat.SIGNATURES, *nat.SIGNATURES_EXT],
+                                                   lambda *a: ran.append(a) or 0))
+    t = torch.zeros(1, 2, 8, 4)
+    with pytest.raises((RuntimeError, ValueError)):
+        nat.stream_of(t)
+    with pytest.raises(RuntimeError, match="cpu"):
+        nat.call("mqc_sum_rows", t, 0)
+    with pytest.raises((RuntimeError, ValueError)):
+        torch.ops.mambaqc.quaternion_layer_norm_backward(t, t[0, 0, :, 0], t[..., 0, 0],
+                                                         t[..., 0, 0], t)
+    assert not ran
