@@ -36,8 +36,8 @@ def _d_strides(D: torch.Tensor, dtype: torch.dtype):
 
 # The time-chunked q form (mqc_ssm_q_fwd_chunked) reads q and B twice, so it pays where the whole
 # walk is bound by its serial chain, 0.4 us a step (us, whole / chunked): fp32 T 4096 1024 lanes
-# 1661 / 84, 8192 1774 / 456, 24576 (T 2000) 843 / 646, but 49152 924 / 1367; bf16 8192 1709 / 251,
-# 49152 (T 2000) 868 / 697; T 150 3200 lanes 63 / 22.
+# 1649 / 80, 8192 1662 / 471, 24576 (T 2000) 821 / 662, but 49152 924 / 1367; bf16 8192 1614 / 268,
+# 49152 (T 2000) 799 / 782; T 150 3200 lanes 62 / 22.
 Q_CHUNK_MAX_BYTES = 96 << 10  # batch x lanes x element size
 Q_CHUNK_MIN_SEQ = 64
 
