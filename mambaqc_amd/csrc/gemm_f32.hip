@@ -26,9 +26,12 @@
 //     (the input gradient's) is blocked too, each block adding to the partial sums; its
 //     blocks are twice as large, since each adds a pass over the partial sums. Measured, blocks of
 //     16 and 32 Mi elements (us): forward M 2048 N 65536 K 512 518 / 600, M 4096 N 98304
-//     K 768 1874 / 2026; input gradients of the two 781 / 711 and 2890 / 2679.
-//   - Few output tiles (the input gradient): k is shared by `splits` workgroups per tile,
-//     whose partial sums a last launch adds in order.
+//     K 768 1874 / 2026; input gradients of the two 781 / 711 and 2890 / 2679. So is a k that
+//     takes the shorter side past one block (the weight gradient of many tokens): that side would
+//     otherwise be split again for every block of the longer one.
+//   - Few output tiles in a block (the input gradient): k is shared by `splits` workgroups per
+//     tile, whose partial sums a last launch adds in order, block by block. They are at most 512 tiles
+//     of 128 x 128 (32 MiB) at a time, whatever the output's size.
 #include <atomic>
 
 #include "mfma_tile.hpp"
@@ -330,16 +333,17 @@ __global__ __launch_bounds__(Cfg::kThreads) void gemm_f32_kernel(GemmF32Args a) 
   }
 }
 
-// Y = the sum of the partial sums, in order of k.
+// A block of Y (+)= the sum of its partial sums, rows of N, in order of k.
 __global__ __launch_bounds__(256) void sum_splits_kernel(const float* __restrict__ part,
                                                          int64_t stride, int splits,
                                                          float* __restrict__ Y, int64_t ldy, int N,
-                                                         int64_t total) {
+                                                         int64_t total, int accumulate) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
+  float* y = Y + i / N * ldy + i % N;
   float s = part[i];
   for (int z = 1; z < splits; ++z) s += part[z * stride + i];
-  Y[i / N * ldy + i % N] = s;
+  *y = accumulate ? *y + s : s;
 }
 
 using Big = Tile256;
@@ -358,11 +362,17 @@ inline int64_t padk(int64_t k) { return up(k, kChunk); }
 
 Plan plan(int64_t M, int64_t N, int64_t K) {
   Plan p;
-  // k is blocked only where it is the long axis (both operands are then read along it).
+  // k is blocked where it is the long axis (both operands are then read along it) or the shorter
+  // side does not fit one block: by 2 kBlockElems / longest, or 8192 where that is less and the shorter
+  // side fits (each block of k passes over the output once more).
   p.kb = K;
-  const int64_t longest = M > N ? M : N;
-  if (K > longest && K * longest > 2 * kBlockElems) {
-    p.kb = up(2 * kBlockElems / longest, 256);
+  const int64_t longest = M > N ? M : N, shortest = M > N ? N : M;
+  if ((K > longest && K * longest > 2 * kBlockElems) || K * shortest > kBlockElems) {
+    int64_t by_short = kBlockElems / up(shortest, 256) / 256 * 256;
+    if (by_short > 8192) by_short = 8192;
+    p.kb = 2 * kBlockElems / longest;
+    if (p.kb < by_short) p.kb = by_short;
+    p.kb = up(p.kb > 0 ? p.kb : 1, 256);
     if (p.kb > K) p.kb = K;
   }
   auto rows = [&](int64_t r) {
@@ -412,7 +422,7 @@ int64_t f32_workspace(int64_t M, int64_t N, int64_t K) {
   const Plan p = plan(M, N, K);
   const int64_t kp = padk(p.kb);
   int64_t b = up(p.mb * kp * 4, 256) + up(p.nb * kp * 4, 256) + max_words(p, M, N, K) * 4;
-  if (p.splits > 1) b += p.splits * M * N * 4;
+  if (p.splits > 1) b += p.splits * p.mb * p.nb * 4;
   return b;
 }
 
@@ -533,13 +543,16 @@ int mqc_gemm_f32(const float* X, int64_t x_row, int64_t x_col, const float* W, i
         a.X = Xb; a.W = Wb; a.xm = x_row; a.xk = x_col; a.wn = w_row; a.wk = w_col;
         a.M = (int)mn; a.N = (int)nn; a.K = (int)kn; a.Kp = (int)padk(kn);
         a.splits = p.splits;
-        a.accumulate = k0 > 0;
+        float* const Yb = Y + m0 * ldy + n0;
+        // (One block of the output keeps its partial sums over the blocks of k.)
+        const bool keeps = p.mb >= M && p.nb >= N;
+        a.accumulate = k0 > 0 && (p.splits == 1 || keeps);
         if (p.splits > 1) {
-          a.out = part + m0 * N + n0;
-          a.ldo = N;
-          a.split_stride = M * N;
+          a.out = part;
+          a.ldo = nn;
+          a.split_stride = p.mb * p.nb;
         } else {
-          a.out = Y + m0 * ldy + n0;
+          a.out = Yb;
           a.ldo = ldy;
         }
         const int t = p.big ? 256 : 128;
@@ -548,16 +561,13 @@ int mqc_gemm_f32(const float* X, int64_t x_row, int64_t x_col, const float* W, i
           gemm_f32_kernel<Big><<<grid, Big::kThreads, Big::kStagesBytes, s>>>(a);
         else
           gemm_f32_kernel<Small><<<grid, Small::kThreads, Small::kStagesBytes, s>>>(a);
+        if (p.splits > 1 && (!keeps || k0 + kn == K))
+          sum_splits_kernel<<<(unsigned)((mn * nn + 255) / 256), 256, 0, s>>>(
+              part, a.split_stride, p.splits, Yb, ldy, (int)nn, mn * nn, k0 > 0 && !keeps);
         st = launch_status();
         if (st != MQC_OK) return st;
       }
     }
-  }
-  if (p.splits > 1) {
-    const int64_t total = M * N;
-    sum_splits_kernel<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(part, M * N, p.splits, Y, ldy,
-                                                                      (int)N, total);
-    return launch_status();
   }
   return MQC_OK;
 }

@@ -40,11 +40,12 @@ def _views(form, M, N, K, g):
 
 
 # Edges of the 128 and 256 tiles, one row, k remainders (a line of pieces holds 32, rows of
-# k past 1024, 2048 and 16384 are read differently), shares of k, blocks of k and of rows.
+# k past 1024, 2048 and 16384 are read differently), shares of k, blocks of k and of rows, and
+# all three together (partial sums added to the output block by block).
 @pytest.mark.parametrize("form", ["nn", "nt", "tt", "tn"])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (129, 127, 33), (257, 300, 64), (64, 65, 1030),
                                    (300, 9000, 70), (5, 40, 2049), (33, 20, 17000),
-                                   (128, 130, 270001), (700, 24000, 1500)])
+                                   (128, 130, 270001), (700, 24000, 1500), (5000, 140, 30000)])
 def test_against_float64(form, M, N, K):
     g = torch.Generator(device="cuda").manual_seed(M * 31 + N * 7 + K)
     x, w = _views(form, M, N, K, g)
