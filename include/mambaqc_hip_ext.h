@@ -11,13 +11,16 @@
 extern "C" {
 #endif
 
-/* fp32 GEMM at fp32 accuracy on the 16-bit matrix cores (each operand split into two fp16
- * pieces under a power-of-two scale per row, three products per pair of pieces, fp32
- * accumulation; rows with an inf or a NaN are computed in plain fp32):
+/* fp32 GEMM on the 16-bit matrix cores (each operand split into two fp16 pieces under a
+ * power-of-two scale per row, three products per pair of pieces, fp32 accumulation):
  *   Y[m * ldy + n] = sum_k X[m * x_row + k * x_col] * W[n * w_row + k * w_col]
  * for m < M, n < N, k < K. One of x_row and x_col and one of w_row and w_col is 1 (and none
  * is negative), so X and W may be matrices or their transposes: F.linear and both of its
  * gradients (mambaqc/layers/quaternion_linear.py:145-161). Y may not overlap an operand.
+ * Accuracy: each element is held to 2^-23 of itself, or to 2^-40 of its row's largest where that
+ * is more; outputs that this last may put off by more than 2^-28 K of themselves (2^-20 below
+ * K 256), all outputs of rows where more than an eighth of the elements are so small, and of
+ * rows with an inf, are computed in plain fp32.
  * workspace: mqc_gemm_f32_workspace_bytes(M, N, K) bytes, 256-byte aligned (MQC_E_SPACE
  * if smaller). */
 int64_t mqc_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);

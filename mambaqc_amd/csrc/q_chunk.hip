@@ -11,15 +11,15 @@
 //      E_c = P_c (x) E_{c-1} (+ H_c);
 //   3. the usual kernels on every chunk from its carry.
 //
-// P is held as a quaternion of magnitude about 1 times 2^X: a chunk of decaying (or growing) q's takes it
-// far past fp32's range, where the carried value itself may be anywhere. What fp32 could not
-// hold on the way, the walk itself would not have held either, or it is marked, and the prefix walks those
-// lanes' chunks step by step from their carry: a q so small or large that P leaves the range
-// within 8 steps, an inf or a NaN, and products that could overflow with the carry at hand. (The bookkeeping
-// costs at most 7 us: cumulative product, T 4096, bf16 1024 lanes 36 without and 44 with it, fp32 4096
-// lanes 138 and 146, the SSM's q form within its noise.)
-// Launch 1 reads q (and B) a second time, so it pays only where the chain, not HBM, is the bound: the
-// rules are with the callers (kernels/parallel_scan.py, kernels/ssm_fused.py), both sides measured.
+// P is held as a quaternion of magnitude about 1 times 2^X: a chunk of decaying (or growing) q's
+// takes it far past fp32's range, where the carried value itself may be anywhere. What fp32 could
+// not hold on the way, the walk itself would not have held either, or it is marked, and the prefix
+// walks those lanes' chunks step by step from their carry: a q so small or large that P leaves the
+// range within 8 steps, an inf or a NaN, and products that could overflow with the carry at hand.
+// (The bookkeeping costs at most 7 us: cumulative product, T 4096, bf16 1024 lanes 36 without and
+// 44 with it, fp32 4096 lanes 138 and 146, the SSM's q form within its noise.) Launch 1 reads q
+// (and B) a second time, so it pays only where the chain, not HBM, is the bound: the rules are with
+// the callers (kernels/parallel_scan.py, kernels/ssm_fused.py), both sides measured.
 #include "ssm_scan.hpp"
 
 namespace mqc {

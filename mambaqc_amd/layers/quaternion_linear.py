@@ -136,15 +136,16 @@ class _WideLinearFunction(torch.autograd.Function):
         return dx, dw, None
 
 
-# fp32 products run on the library's split-fp16 GEMM (mqc_gemm_f32: fp32 accuracy on the
-# 16-bit matrix cores) where it is the faster one. Against hipBLASLt's fp32, which reaches
-# 115-153 of the fp32 matrix cores' 157 TFLOP/s, it multiplies at 300-380 TFLOP/s but first
-# splits both operands (8 bytes moved per element), so the shorter side of the product has to
-# repay that, and the whole one its extra launches. Measured on MI355X (us, library / this
-# GEMM): forward M 1024 N 131072 K 1024 1935 / 954, M 400 N 32768 K 512 129 / 75; input
-# gradients of the same 2223 / 1329 and 358 / 135; weight gradients 1912 / 1132 and 110 / 87.
-# Below the line: M 100 N 98304 K 384 86 / 120 (a short side), 98304 x 384 over K 100
-# 94 / 114 (short k: padding and output dominate), 1024 x 1024 x 1024 22 / 35 (launches).
+# fp32 products run on the library's split-fp16 GEMM (mqc_gemm_f32: fp32 operands as pairs of
+# fp16 pieces on the 16-bit matrix cores, what the pieces do not hold in plain fp32) where it is
+# the faster one. Against hipBLASLt's fp32, which reaches 115-153 of the fp32 matrix cores' 157
+# TFLOP/s, it multiplies at 300-380 TFLOP/s but first splits both operands (8 bytes moved per
+# element), so the shorter side of the product has to repay that, and the whole one its extra
+# launches. Measured on MI355X (us, library / this GEMM): forward M 1024 N 131072 K 1024
+# 1940 / 915, M 400 N 32768 K 512 131 / 81; input gradients of the same 2230 / 2100 and 359 / 137;
+# weight gradients 1990 / 1174 and 105 / 94. Below the line: M 100 N 98304 K 384 86 / 120 (a
+# short side), 98304 x 384 over K 100 94 / 114 (short k: padding and output dominate), 1024 x 1024
+# x 1024 22 / 35 (launches).
 F32_GEMM_MIN_SIDE = 200     # M N / (M + N)
 F32_GEMM_MIN_K = 192
 F32_GEMM_MIN_FLOP = 6e9

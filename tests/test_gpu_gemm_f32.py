@@ -23,13 +23,12 @@ def _gemm(x, w):
 
 def _bound(x, w):
     """Elementwise: what the split drops (lo lo <= 2^-22 of a product, each lo rounded to
-    2^-23 of its value, or 2^-39 of its row's largest), and the fp32 roundings of an
-    accumulator that takes 3 MFMAs per 32 k plus the partial sums."""
+    2^-23 of its value), what elements far below their row's largest lose (2^-28 K of an
+    output, 2^-20 below K 256, or it is computed again), and the fp32 roundings of an accumulator that takes 3 MFMAs per
+    32 k plus the partial sums, or of a product computed again, 4 k per rounding."""
     K = x.shape[1]
-    xa, wa = x.double().abs(), w.double().abs()
-    prod = xa @ wa.t()
-    floor = K * 2.0 ** -38 * xa.amax(1, keepdim=True) * wa.amax(1).unsqueeze(0)
-    return (2.0 ** -21 + (3 * K / 32 + 72) * 2.0 ** -24) * prod + floor
+    prod = x.double().abs() @ w.double().abs().t()
+    return (2.0 ** -21 + max(K, 256) * 2.0 ** -28 + (K / 4 + 72) * 2.0 ** -24) * prod
 
 
 def _views(form, M, N, K, g):
@@ -85,6 +84,67 @@ def test_magnitudes_and_non_finite_rows(form):
     assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf())
     assert torch.equal(y[y.isinf()], ref[ref.isinf()])
     assert y[~bad].isfinite().all()
+
+
+def _wide(kind, big, a, g):
+    """a [R, K] with elements of size `big` in some columns (returned)."""
+    cols = {"one": slice(3, 4), "half": slice(0, None, 2), "all but one": slice(1, None),
+            "some rows": slice(5, 6)}[kind]
+    rows = slice(0, None, 3) if kind == "some rows" else slice(None)
+    a[rows, cols] = big * torch.rand(a[rows, cols].shape, generator=g, device="cuda").add_(0.5)
+    return cols
+
+
+@pytest.mark.parametrize("form", ["nn", "tt"])
+@pytest.mark.parametrize("side", ["x", "w"])
+@pytest.mark.parametrize("big", [1e3, 1e4, 1e5, 1e6, 1e7, 1e9, 1e13, 1e30])
+def test_rows_of_wide_range(form, side, big):
+    """Columns far above the rest that the other operand's zeros leave out (an outlier feature, a
+    masked sentinel, one token's gradient): what counts is at 2^-10 to 2^-100 of its row's
+    largest, and the error is the fp32 library's all the same. (An output that is one product, of
+    one small element: within the bound above for what is not computed again.)"""
+    g = torch.Generator(device="cuda").manual_seed(int(big) % 1000)
+    for kind in ("one", "half", "all but one", "some rows"):
+        for M, N, K in ((150, 200, 512), (40, 300, 2000)):
+            x, w = _views(form, M, N, K, g)
+            a, o = (x, w) if side == "x" else (w, x)
+            o[:, _wide(kind, big, a, g)] = 0.0
+            y, lib, ref = _gemm(x, w), x @ w.t(), x.double() @ w.double().t()
+            assert ((y.double() - ref).abs() <= _bound(x, w)).all(), (kind, M, N, K)
+            err, lib_err = ((v.double() - ref).norm() / ref.norm() for v in (y, lib))
+            least = K * 2.0 ** -28 if kind == "all but one" else 2.0 ** -22
+            assert err <= max(1.2 * lib_err.item(), least), (kind, K, err.item(), lib_err.item())
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tt", "tn"])
+def test_listed_rows_among_others(form):
+    """Lists of none, of one, of a few, past a tile of them and of all rows, on both sides and
+    over blocks of k, with ragged sizes; a listed row's outputs are the same whatever else is."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    for M, N, K in ((70, 67, 203), (33, 130, 64), (1200, 140, 30000)):
+        x, w = _views(form, M, N, K, g)
+        first = None
+        for nx, nw in ((1, 0), (1, 1), (33, 5), (0, 64), (M, N)):
+            xs, ws = x.clone(), w.clone()
+            xs[:nx, K - 1], ws[N - nw:, 0] = 1e8, -1e9
+            y, ref = _gemm(xs, ws), xs.double() @ ws.double().t()
+            assert ((y.double() - ref).abs() <= _bound(xs, ws)).all(), (M, N, K, nx, nw)
+            if nx and not nw:
+                first = y[0].clone()
+            elif nx:
+                assert torch.equal(y[0, :N - nw], first[:N - nw])
+
+
+def test_every_row_with_an_inf():
+    """One inf in x puts one in every row of its transpose."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    for form in ("nn", "tt"):
+        x, w = _views(form, 300, 500, 700, g)
+        x[:, 11] = float("inf")
+        w[7, 11] = 0.0
+        y, ref = _gemm(x, w), x @ w.t()
+        assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf())
+        assert torch.equal(y[y.isinf()], ref[ref.isinf()])
 
 
 def test_wide_linear_takes_it_with_gradients_of_gradients():
