@@ -32,11 +32,12 @@
 //   - Blocks: an operand is split a block at a time (kBlockElems, 64 MiB of pieces), and each
 //     block is multiplied while its pieces are still in the 256 MiB Infinity Cache. Long k
 //     (the input gradient's) is blocked too, each block adding to the partial sums; its
-//     blocks are twice as large, since each adds a pass over the partial sums. Measured, blocks of
-//     16 and 32 Mi elements (us): forward M 2048 N 65536 K 512 518 / 600, M 4096 N 98304
-//     K 768 1874 / 2026; input gradients of the two 781 / 711 and 2890 / 2679. So is a k that
-//     takes the shorter side past one block (the weight gradient of many tokens): that side would
-//     otherwise be split again for every block of the longer one.
+//     blocks are twice as large, since each adds a pass over the partial sums and one of half the
+//     rows splits the other operand again. Measured, blocks of 16 and 32 Mi elements (us): forward
+//     M 2048 N 65536 K 512 518 / 600, M 4096 N 98304 K 768 1874 / 2026; input gradients
+//     M 2048 N 512 K 65536 777 / 711, M 4096 N 768 K 98304 2960 / 2738, M 1024 N 1024 K 131072
+//     2239 / 1436, M 600 N 384 K 98304 1327 / 598. So is a k that takes the shorter side past one
+//     block (the weight gradient of many tokens), for the same reason.
 //   - Few output tiles in a block (the input gradient): k is shared by `splits` workgroups per
 //     tile, whose partial sums a last launch adds in order, block by block. They are at most 512
 //     tiles of 128 x 128 (32 MiB) at a time, whatever the output's size.
@@ -667,6 +668,7 @@ Plan plan(int64_t M, int64_t N, int64_t K) {
   // side does not fit one block: by 2 kBlockElems / longest, or 8192 where that is less and the
   // shorter side fits (each block of k passes over the output once more).
   p.kb = K;
+  int64_t elems = kBlockElems;
   const int64_t longest = M > N ? M : N, shortest = M > N ? N : M;
   if ((K > longest && K * longest > 2 * kBlockElems) || K * shortest > kBlockElems) {
     int64_t by_short = kBlockElems / up(shortest, 256) / 256 * 256;
@@ -675,9 +677,10 @@ Plan plan(int64_t M, int64_t N, int64_t K) {
     if (p.kb < by_short) p.kb = by_short;
     p.kb = up(p.kb > 0 ? p.kb : 1, 256);
     if (p.kb > K) p.kb = K;
+    if (K > longest) elems = 2 * kBlockElems;
   }
   auto rows = [&](int64_t r) {
-    int64_t most = kBlockElems / padk(p.kb) / 256 * 256;
+    int64_t most = elems / padk(p.kb) / 256 * 256;
     if (most < 256) most = 256;
     return r < most ? r : most;
   };

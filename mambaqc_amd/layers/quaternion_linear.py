@@ -142,7 +142,7 @@ class _WideLinearFunction(torch.autograd.Function):
 # TFLOP/s, it multiplies at 300-380 TFLOP/s but first splits both operands (8 bytes moved per
 # element), so the shorter side of the product has to repay that, and the whole one its extra
 # launches. Measured on MI355X (us, library / this GEMM): forward M 1024 N 131072 K 1024
-# 1940 / 915, M 400 N 32768 K 512 131 / 81; input gradients of the same 2230 / 2100 and 359 / 137;
+# 1940 / 915, M 400 N 32768 K 512 131 / 81; input gradients of the same 2290 / 1436 and 358 / 138;
 # weight gradients 1990 / 1174 and 105 / 94. Below the line: M 100 N 98304 K 384 86 / 120 (a
 # short side), 98304 x 384 over K 100 94 / 114 (short k: padding and output dominate), 1024 x 1024
 # x 1024 22 / 35 (launches).

@@ -342,14 +342,14 @@ def test_gemm_validation_without_gpu():
 
 
 def test_gemm_f32_workspace_is_bounded():
-    """Pieces of two blocks and the partial sums of one, for any number of tokens: a weight
-    gradient's k is its tokens, a forward's rows are."""
+    """Pieces of two blocks (at most 128 MiB each) and the partial sums of one, for any number of
+    tokens: a weight gradient's k is its tokens, a forward's rows are."""
     lib = nat.load()
     for m in (200, 1000, 4096, 131072, 393216):
         for n in (200, 512, 1024, 3072, 131072):
             for k in (192, 1024, 8192, 16384, 32768, 65536, 131072):
                 need = lib.mqc_gemm_f32_workspace_bytes(m, n, k)
-                assert 0 < need <= max(256 << 20, m * n * 4 // 32), (m, n, k, need)
+                assert 0 < need <= max(320 << 20, m * n * 4 // 32), (m, n, k, need)
 
 
 def test_step_counter_limits_without_gpu():
