@@ -675,10 +675,12 @@ Plan plan(int64_t M, int64_t N, int64_t K) {
     if (by_short > 8192) by_short = 8192;
     p.kb = 2 * kBlockElems / longest;
     if (p.kb < by_short) p.kb = by_short;
-    p.kb = up(p.kb > 0 ? p.kb : 1, 256);
+    // (Of equal length, or the last one's launches would be mostly overhead.)
+    const int64_t blocks = p.kb > 0 ? (K + p.kb - 1) / p.kb : K;
+    p.kb = up((K + blocks - 1) / blocks, 256);
     if (p.kb > K) p.kb = K;
-    if (K > longest) elems = 2 * kBlockElems;
   }
+  if (K > longest) elems = 2 * kBlockElems;
   auto rows = [&](int64_t r) {
     int64_t most = elems / padk(p.kb) / 256 * 256;
     if (most < 256) most = 256;
@@ -698,9 +700,11 @@ Plan plan(int64_t M, int64_t N, int64_t K) {
   rounds(p.mb, M, p.nb);
   const int64_t t256 = ((p.mb + 255) / 256) * ((p.nb + 255) / 256);
   const int64_t t128 = ((p.mb + 127) / 128) * ((p.nb + 127) / 128);
-  // The 128 x 128 tile where one side is short (a 256-row tile would be mostly padding) or
-  // the 256 x 256 tiles would leave CUs idle.
-  p.big = p.mb > 128 && p.nb > 128 && t256 >= kCUsF * 3 / 4;
+  // The 128 x 128 tile where one side is short or rows of X would be padding (M 273 N 73728 K 384
+  // 167 / 136 us; padding of W's rows costs less than the smaller tile does, M 30720 N 320 K 534
+  // 104 / 114), or the 256 x 256 tiles would leave CUs idle.
+  p.big = p.mb > 128 && p.nb > 128 && up(p.mb, 256) * 8 <= up(p.mb, 128) * 9 &&
+          t256 >= kCUsF * 3 / 4;
   const int64_t tiles = p.big ? t256 : t128;
   const int64_t slots = p.big ? kCUsF : 2 * kCUsF;  // workgroups resident at once
   const int64_t steps = padk(p.kb) / kChunk;
