@@ -143,17 +143,35 @@ class _WideLinearFunction(torch.autograd.Function):
 # element), so the shorter side of the product has to repay that, and the whole one its extra
 # launches. Measured on MI355X (us, library / this GEMM): forward M 1024 N 131072 K 1024
 # 1940 / 915, M 400 N 32768 K 512 131 / 81; input gradients of the same 2290 / 1436 and 358 / 138;
-# weight gradients 1990 / 1174 and 105 / 94. Below the line: M 100 N 98304 K 384 86 / 120 (a
-# short side), 98304 x 384 over K 100 94 / 114 (short k: padding and output dominate), 1024 x 1024
-# x 1024 22 / 35 (launches).
-F32_GEMM_MIN_SIDE = 200     # M N / (M + N)
+# weight gradients 1990 / 1174 and 105 / 94. Below the lines: M 100 N 98304 K 384 86 / 120 (a short
+# side), 98304 x 384 over K 100 94 / 114 (short k: padding and output dominate), 1024 x 1024 x 1024
+# 22 / 35 (launches). An operand with its rows contiguous is read once more for the rows' maxima, so
+# the side that repays it is longer: with none (a forward) M 255 N 294912 K 1536 1622 / 1922, M 306
+# N 196608 K 768 737 / 666; with one (an input gradient) M 1602 N 320 K 51200 419 / 541, M 639 N 768
+# K 49152 432 / 456, M 1212 N 512 K 40960 481 / 352; with two (a weight gradient) M 49152 N 256 K 2203
+# 406 / 648, M 98304 N 384 K 5679 2878 / 3627, M 30720 N 384 K 5286 1132 / 970, M 98304 N 512 K 2427
+# 1717 / 1722, M 51200 N 640 K 523 270 / 236. An input gradient of few outputs leaves the library's
+# GEMM at 40-80 TFLOP/s and pays at any side from 200 on (M 973 N 256 K 24576 324 / 130, M 574 N 384
+# K 36864 327 / 199).
+F32_GEMM_MIN_SIDE = (256, 350, 500)  # M N / (M + N), by the operands with their rows contiguous
+F32_GEMM_FEW_OUTPUTS = 300_000       # up to this many, with one such operand at most:
+F32_GEMM_FEW_MIN_SIDE = 200
 F32_GEMM_MIN_K = 192
 F32_GEMM_MIN_FLOP = 6e9
 
 
-def _f32_gemm_shape(M: int, N: int, K: int) -> bool:
-    return (K >= F32_GEMM_MIN_K and M * N >= F32_GEMM_MIN_SIDE * (M + N)
+def _f32_gemm_shape(M: int, N: int, K: int, by_rows: int = 0) -> bool:
+    """Whether an fp32 product runs on mqc_gemm_f32, `by_rows` of its operands having their rows
+    and not k contiguous."""
+    side = F32_GEMM_MIN_SIDE[by_rows]
+    if by_rows < 2 and M * N <= F32_GEMM_FEW_OUTPUTS:
+        side = min(side, F32_GEMM_FEW_MIN_SIDE)
+    return (K >= F32_GEMM_MIN_K and M * N >= side * (M + N)
             and 2.0 * M * N * K >= F32_GEMM_MIN_FLOP)
+
+
+def _by_rows(t: torch.Tensor) -> bool:
+    return t.dim() == 2 and t.stride(0) == 1 and t.stride(1) != 1
 
 
 def _unit_rows(t: torch.Tensor) -> torch.Tensor:
@@ -187,7 +205,8 @@ def _f32_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
 def _f32_eligible(x: torch.Tensor, w: torch.Tensor, rows: int) -> bool:
     """Whether x w^T, x of `rows` rows, runs on mqc_gemm_f32."""
     n, k = w.shape
-    return (_f32_operands(x, w) and _f32_gemm_shape(rows, n, k) and _plain_call(x, w)
+    return (_f32_operands(x, w) and _f32_gemm_shape(rows, n, k, _by_rows(x) + _by_rows(w))
+            and _plain_call(x, w)
             and not torch.is_autocast_enabled(x.device.type))
 
 

@@ -36,7 +36,7 @@ def launches(monkeypatch):
 
     monkeypatch.setattr(nat, "call", call)
     monkeypatch.setattr(nat, "stream_of", lambda t: 0)
-    monkeypatch.setattr(ql, "_f32_gemm_shape", lambda M, N, K: True)
+    monkeypatch.setattr(ql, "_f32_gemm_shape", lambda *a: True)
     monkeypatch.setattr(ql, "_f32_operands", lambda x, w: x.dtype == w.dtype == torch.float32,
                         raising=False)
     return seen
@@ -263,3 +263,17 @@ def test_host_tensors_never_reach_a_launch(monkeypatch):
         torch.ops.mambaqc.quaternion_layer_norm_backward(t, t[0, 0, :, 0], t[..., 0, 0],
                                                          t[..., 0, 0], t)
     assert not ran
+
+
+def test_fp32_gemm_sizes():
+    """Both sides of the lines that the sizes were measured at, by the operands' layouts."""
+    takes = ql._f32_gemm_shape
+    assert takes(1024, 131072, 1024) and takes(400, 32768, 512) and takes(306, 196608, 768)
+    assert not takes(255, 294912, 1536) and not takes(100, 98304, 384)
+    assert not takes(98304, 384, 100) and not takes(1024, 1024, 1024)
+    assert takes(1024, 1024, 131072, 1) and takes(400, 512, 32768, 1) and takes(574, 384, 36864, 1)
+    assert not takes(1602, 320, 51200, 1) and not takes(639, 768, 49152, 1)
+    assert takes(131072, 1024, 1024, 2) and takes(32768, 512, 400, 2)
+    assert not takes(49152, 256, 2203, 2) and not takes(98304, 384, 5679, 2)
+    x, w = torch.randn(6, 5), torch.randn(7, 5)
+    assert not ql._by_rows(x) and ql._by_rows(w.t()) and not ql._by_rows(x.view(2, 3, 5))
