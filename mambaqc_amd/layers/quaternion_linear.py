@@ -268,16 +268,30 @@ def _f32_linear_eligible(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return x.shape[-1] == k and _f32_eligible(x, weight, x.numel() // k if k else 0)
 
 
-# Small fp32 products of inference: torch's dispatch of one hipBLASLt fp32 GEMM takes 21 us of
-# host time whatever its size, mqc_gemm_f32_small about 8 for up to four. At this many FLOP and
-# this long a k the GPU is no slower with it (400 x 1024 x 256, 0.2 GFLOP: 9 us, hipBLASLt 10);
-# longer k or more work belongs to kernels that split k or fill the chip.
-F32_SMALL_MAX_FLOP = 6e8
-F32_SMALL_MAX_K = 2048
+# Small fp32 products of inference: torch's dispatch of one hipBLASLt fp32 GEMM takes 19-21 us of
+# host time whatever its size, mqc_gemm_f32_small about 9 for up to four, so a program of small
+# products is bound by the host. On the GPU the kernel has one chain of k per tile (us in a captured
+# graph, library / this one, 64 rows: 256 columns of k 64 7.9 / 3.9, 1024 of 256 6.0 / 8.1, 2048 of
+# 512 8.8 / 13, 3072 of 768 10 / 23, 256 of 2048 8.5 / 43) and streams weights at 2 TB/s. So k is
+# bounded by what the host takes (eager, one product of k 512 20 / 13, two of 1024 39 / 29; one of
+# 768 20 / 22), the weights too (16384 x 512 21 / 28), and the work by where both take about as long
+# on the GPU (400 x 1024 x 256, 0.2 GFLOP, 10 / 9; 200 x 16384 x 64, 0.4 GFLOP, 11 / 17). The few
+# rows of a decode step, which a program captures in a graph where host time is nothing, keep the
+# library beyond k 64 (1 row, 1024 columns: 3.9 / 4.1, of k 256 4.3 / 7.6; 2048 of 2048 12 / 52) and,
+# where one launch takes several, k 256 (four of k 128, 16640 columns, 24 / 12; two of k 1024
+# 17 / 24).
+F32_SMALL_MAX_FLOP = 3e8
+F32_SMALL_MAX_K = (512, 1024)        # for one product in the launch, for several
+F32_SMALL_FEW_ROWS = 32              # below this many rows:
+F32_SMALL_FEW_ROWS_MAX_K = (64, 256)
+F32_SMALL_MAX_WEIGHT_BYTES = 16 << 20  # per product
 
 
-def _f32_small_shape(M: int, N: int, K: int) -> bool:
-    return M > 0 and N > 0 and 0 < K <= F32_SMALL_MAX_K and 2.0 * M * N * K <= F32_SMALL_MAX_FLOP
+def _f32_small_shape(M: int, N: int, K: int, count: int = 1) -> bool:
+    """Whether `count` products of M rows and N columns together run on mqc_gemm_f32_small."""
+    max_k = (F32_SMALL_MAX_K if M >= F32_SMALL_FEW_ROWS else F32_SMALL_FEW_ROWS_MAX_K)[count > 1]
+    return (M > 0 and N > 0 and 0 < K <= max_k and 2.0 * M * N * K <= F32_SMALL_MAX_FLOP
+            and 4 * N * K <= count * F32_SMALL_MAX_WEIGHT_BYTES)
 
 
 def _f32_small_launch(x: torch.Tensor, params, out) -> None:
@@ -315,7 +329,8 @@ def f32_small_eligible(x: torch.Tensor, *params) -> bool:
                               or (grad and b.requires_grad)):
             return False
         columns += w.shape[0]
-    return (_f32_small_shape(rows, columns, K) and not torch.is_autocast_enabled(x.device.type)
+    return (_f32_small_shape(rows, columns, K, len(params) // 2)
+            and not torch.is_autocast_enabled(x.device.type)
             and _plain_call(x, *(p for p in params if p is not None)))
 
 

@@ -277,3 +277,15 @@ def test_fp32_gemm_sizes():
     assert not takes(49152, 256, 2203, 2) and not takes(98304, 384, 5679, 2)
     x, w = torch.randn(6, 5), torch.randn(7, 5)
     assert not ql._by_rows(x) and ql._by_rows(w.t()) and not ql._by_rows(x.view(2, 3, 5))
+
+
+def test_small_fp32_sizes():
+    """A launch's work, weights and k, and the few rows of a decode step."""
+    takes = ql._f32_small_shape
+    assert takes(64, 256, 64) and takes(64, 2 * 128 + 2 * 8192, 128, 4) and takes(64, 64, 512)
+    assert takes(64, 2048, 1024, 2) and not takes(64, 1024, 1024) and not takes(64, 256, 2048)
+    assert not takes(200, 16384, 64) and not takes(64, 16384, 512) and not takes(0, 256, 64)
+    for rows in (1, 4, 16):
+        assert takes(rows, 256, 64) and takes(rows, 2 * 128 + 2 * 8192, 128, 4)
+        assert not takes(rows, 1024, 256) and not takes(rows, 3072, 1536, 2)
+        assert not takes(rows, 2048, 2048) and not takes(rows, 262144, 1024, 2)
