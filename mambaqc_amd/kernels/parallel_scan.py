@@ -17,9 +17,10 @@ from .. import _native as nat
 # The time-chunked product (mqc_cumprod_scan_chunked) reads q twice, so it pays where the whole
 # walk is bound by its serial chain (us, whole / chunked): fp32 T 4096 1024 lanes 182 / 55, 4096
 # 188 / 146, but 8192 263 / 318; bf16 1024 433 / 44, 24576 (T 2000) 379 / 218, 16000 (T 256)
-# 30 / 25, 49152 (T 2000) 463 / 430.
+# 30 / 25, 49152 (T 2000) 463 / 430. Short sequences leave little to save: bf16 T 128 12 / 17,
+# 192 16 / 17, 256 21 / 18, fp32 T 512 24 / 19.
 CHUNK_MAX_LANES = {4: 4096, 2: 24576}   # batch x lanes, by element size
-CHUNK_MIN_SEQ = {4: 512, 2: 128}
+CHUNK_MIN_SEQ = {4: 512, 2: 256}
 
 
 def _chunk_len(B: int, T: int, lanes: int, el: int) -> int:

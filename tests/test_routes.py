@@ -15,6 +15,8 @@ import mambaqc_amd.layers.quaternion_linear as ql
 from mambaqc_amd import _native as nat
 from mambaqc_amd import block
 from mambaqc_amd import kernels as K
+from mambaqc_amd.kernels import parallel_scan as ps
+from mambaqc_amd.kernels import ssm_fused as sf
 
 
 def _at(ptr, r, c, rs, cs):
@@ -289,3 +291,14 @@ def test_small_fp32_sizes():
         assert takes(rows, 256, 64) and takes(rows, 2 * 128 + 2 * 8192, 128, 4)
         assert not takes(rows, 1024, 256) and not takes(rows, 3072, 1536, 2)
         assert not takes(rows, 2048, 2048) and not takes(rows, 262144, 1024, 2)
+
+
+def test_chunked_scan_sizes():
+    """Both sides of the lines on lanes and steps, and no chunks for another element size."""
+    for el, short, long in ((4, 511, 512), (2, 255, 256)):
+        assert not ps._chunk_len(1, short, 1024, el) and ps._chunk_len(1, long, 1024, el)
+    assert ps._chunk_len(1, 4096, 4096, 4) and not ps._chunk_len(1, 4096, 4097, 4)
+    assert sf._q_chunk_len(1, 64, 12288, 4) and not sf._q_chunk_len(1, 64, 24576, 4)
+    assert sf._q_chunk_len(1, 128, 24576, 4) and not sf._q_chunk_len(1, 4096, 24577, 4)
+    assert sf._q_chunk_len(1, 64, 24576, 2) and not sf._q_chunk_len(2, 383, 24576, 2)
+    assert sf._q_chunk_len(2, 384, 24576, 2) and not sf._q_chunk_len(1, 600, 64, 8)
