@@ -48,6 +48,18 @@ class _QLNFunction(torch.autograd.Function):
         return dq, dgamma.to(t_gamma), dbeta.to(t_beta), None
 
 
+# The backward that sums its parameter gradients (mqc_qln_bwd_sums) gives a row 256 threads, so
+# many narrow rows leave most of them idle (us, separate sums / inside, fp32): d 64 16384 rows
+# 47 / 34, 100000 113 / 209, d 128 100000 211 / 233, d 192 300000 767 / 750, d 1024 2000 (bf16)
+# 52 / 20.
+SUMS_MANY_ROWS = 16384
+SUMS_MIN_WIDTH = 192  # above that many rows
+
+
+def _sums_inside(rows: int, d: int) -> bool:
+    return rows > 0 and d > 0 and (rows <= SUMS_MANY_ROWS or d >= SUMS_MIN_WIDTH)
+
+
 def _qln_backward(qc, g, mean, rstd, dout, eps):
     """(dq in q's dtype, dgamma [D] and dbeta [D, 4] in fp32) from the forward's
     operands (q in the kernel's form, gamma fp32) and statistics."""
@@ -55,7 +67,7 @@ def _qln_backward(qc, g, mean, rstd, dout, eps):
     dout = nat.aligned16(dout.to(qc.dtype))
     dq = torch.empty_like(qc)
     rows = B * T
-    nbytes = nat.load().mqc_qln_bwd_sums_workspace_bytes(rows, D) if rows and D else -1
+    nbytes = nat.load().mqc_qln_bwd_sums_workspace_bytes(rows, D) if _sums_inside(rows, D) else -1
     if nbytes > 0:
         # dgamma and dbeta summed inside (d_model up to 4096).
         ws = torch.empty(nbytes, device=qc.device, dtype=torch.uint8)

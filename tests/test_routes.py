@@ -2,6 +2,7 @@
 CPU: an fp32 product's launch is emulated from the pointers that the host code hands over, and
 calls that end in the library's host code run it."""
 import ctypes
+import importlib
 
 import numpy as np
 import pytest
@@ -302,3 +303,9 @@ def test_chunked_scan_sizes():
     assert sf._q_chunk_len(1, 128, 24576, 4) and not sf._q_chunk_len(1, 4096, 24577, 4)
     assert sf._q_chunk_len(1, 64, 24576, 2) and not sf._q_chunk_len(2, 383, 24576, 2)
     assert sf._q_chunk_len(2, 384, 24576, 2) and not sf._q_chunk_len(1, 600, 64, 8)
+
+
+def test_layernorm_backward_sizes():
+    qn = importlib.import_module("mambaqc_amd.kernels.quaternion_norm")
+    assert qn._sums_inside(16384, 8) and qn._sums_inside(300000, 192)
+    assert not qn._sums_inside(16385, 191) and not qn._sums_inside(0, 64)
