@@ -196,9 +196,8 @@ BC_SLICE_BYTES = 2 << 30
 # Inference in bf16 or fp16 from this many tokens per sequence on: the B/C projections and the
 # SSM run as one kernel (mqc_ssm_fused_bc_fwd), B and C computed in 256-token tiles on
 # chip and never stored. Shorter sequences run fused where fused_bc_short_wins says so
-# (kernels/ssm_fused.py), and a batch of one from 129 tokens too (block forward_with_state,
-# fused / unfused: d_model 768, 64 states, T 200 740 / 780 us, 255 767 / 819; d_model 512, 32 states T 200
-# 258 / 312; two sequences of 129 to 255 tokens keep the GEMMs, 1200 / 780). A batch of one runs the kernel with
+# (kernels/ssm_fused.py; two sequences of 129 to 255 tokens keep the GEMMs, 1200 fused and 780 us at
+# d_model 768, 64 states, T 200). A batch of one runs the kernel with
 # each half of the states in a workgroup of its own (ssm_forward_fused_bc's split), since
 # one workgroup per d would re-stream more weight rows than the Infinity Cache holds.
 # Block forward at the config-3 width, fused against unfused (one box): B1 T2048 4.63 /
@@ -410,7 +409,7 @@ class QuaternionMamba2Block(nn.Module):
     projections fused into the SSM kernel (ssm_forward_fused_bc) where that
     kernel applies (bf16 or fp16 operands, or autocast to either; bias-free
     projections, d_inner a multiple of 64, even d_state <= 64) and sequences have at least
-    FUSED_BC_MIN_SEQ tokens, or fewer where that is still faster (_fused_bc_short); True
+    FUSED_BC_MIN_SEQ tokens, or fewer where that is still faster (fused_bc_short_wins); True
     also for all other short ones; False never. A forced bc_slice_d takes precedence.
 
     fuse_out (attribute): True runs the output step of bf16 inference (out_proj,
@@ -659,18 +658,12 @@ class QuaternionMamba2Block(nn.Module):
             return False
         if self.B_proj.bias is not None or self.C_proj.bias is not None:
             return False
-        if self.fuse_bc is None and x.shape[1] < FUSED_BC_MIN_SEQ and not self._fused_bc_short(x):
+        if (self.fuse_bc is None and x.shape[1] < FUSED_BC_MIN_SEQ
+                and not _sf.fused_bc_short_wins(*x.shape, self.d_state)):
             return False
         dt = (torch.get_autocast_dtype(x.device.type)
               if torch.is_autocast_enabled(x.device.type) else None)
         return fused_bc_eligible(x, self.B_proj.weight, self.C_proj.weight, self.d_state, dt)
-
-    def _fused_bc_short(self, x: torch.Tensor) -> bool:
-        """Whether sequences below FUSED_BC_MIN_SEQ still run fused."""
-        b, t, D = x.shape
-        if t > _sf.FUSED_BC_SHORT_MAX_SEQ:
-            return b == 1
-        return _sf.fused_bc_short_wins(b, t, D, self.d_state)
 
     def _gemm_dtype(self, x: torch.Tensor) -> torch.dtype:
         if torch.is_autocast_enabled(x.device.type):

@@ -545,22 +545,40 @@ FUSED_BC_SHORT_MAX_SEQ = 128
 # batch every weight row is read once, and the short form is the faster one: d_inner 1536, 64
 # states, batch 1 x 17 tokens 410 / 503, x 64 454 / 572, x 100 514 / 633, x 128 544 / 656,
 # 2 x 64 539 / 632; d_inner 512 x 64 states 1 x 100 66 / 117. Several tiles each stream the weights
-# through L2 again where the GEMM shares them: 2 x 100 788 / 666, 4 x 64 812 / 686, and at d_inner 1024,
-# 32 states (512 MiB of weights) 191 / 201 and 194 / 196. Weights that fit the Infinity Cache together
-# still win: d_inner 512, 64 states (256 MiB) 4 x 64 115 / 140, 4 x 100 223 / 218, 4 x 128 227 / 267;
-# 16 states 4 x 128 59 / 92. Up to 16 rows the decode projections (skinny GEMM) stream the weights at HBM speed
-# already.
+# through L2 again where the GEMM shares them: 2 x 100 788 / 666, 4 x 64 812 / 686, and at d_inner
+# 1024, 32 states (512 MiB of weights) 191 / 201 and 194 / 196. Weights that fit the Infinity Cache
+# together still win in a few tiles: d_inner 512, 64 states (256 MiB) 4 x 64 115 / 140, 4 x 100
+# 223 / 218, 4 x 128 227 / 267; 16 states 4 x 128 59 / 92; but (whole block) d_inner 512, 64 states
+# 16 x 33 (6 tiles) 369 / 333, d_inner 768, 24 states 6 x 100 352 / 303, d_inner 1024, 16 states
+# 16 x 100 714 / 595. Up to 16 rows the decode projections (skinny GEMM) stream the weights at HBM
+# speed already.
 FUSED_BC_SHORT_MIN_ROWS = 17
 FUSED_BC_SHORT_CACHED_BYTES = 256 << 20
+FUSED_BC_SHORT_MAX_TILES = 4
+# A batch of one with 129 to 255 tokens takes the 256-token tile, 32 states to a workgroup, whose
+# time does not depend on how full either is (block forward_with_state, fused / unfused, us):
+# d_inner 1536, 64 states, 129 tokens 738 / 700, 160 742 / 772, 255 761 / 818; 32 states 129 412 /
+# 415, 255 411 / 468; 48 states 129 696 / 627; 16 states 255 374 / 349; d_inner 768, 16 states 129
+# 139 / 149, 48 254 / 297, 40 248 / 229; d_inner 512, 40 states 129 141 / 180.
+FUSED_BC_ONE_MIN_SEQ = 160       # whole groups of 32 states, more than one
+FUSED_BC_ONE_ANY_WIDTH = 512     # up to this d_inner any number of states,
+FUSED_BC_ONE_HALF_WIDTH = 768    # up to this one whole groups of 16
 
 
 def fused_bc_short_wins(batch: int, seq_len: int, d_inner: int, d_state: int) -> bool:
-    """Whether the fused short form beats separate projections for these sizes (of at most
-    FUSED_BC_SHORT_MAX_SEQ tokens; 16-bit operands)."""
-    if not 0 < seq_len <= FUSED_BC_SHORT_MAX_SEQ or batch * seq_len < FUSED_BC_SHORT_MIN_ROWS:
+    """Whether the fused form beats separate projections for these sizes (of fewer than 256
+    tokens; 16-bit operands)."""
+    if seq_len < 1 or batch * seq_len < FUSED_BC_SHORT_MIN_ROWS:
         return False
-    one_tile = batch * (-(-seq_len // 8) * 8) <= 128
-    return one_tile or 2 * d_inner * d_state * 4 * d_inner * 2 <= FUSED_BC_SHORT_CACHED_BYTES
+    if seq_len > FUSED_BC_SHORT_MAX_SEQ:
+        return batch == 1 and (
+            d_inner <= FUSED_BC_ONE_ANY_WIDTH
+            or d_inner <= FUSED_BC_ONE_HALF_WIDTH and d_state % 16 == 0
+            or d_state == 32 or d_state % 32 == 0 and seq_len >= FUSED_BC_ONE_MIN_SEQ)
+    per_tile = 128 // (-(-seq_len // 8) * 8)  # sequences, each in whole chunks of 8 tokens
+    tiles = -(-batch // per_tile)
+    return tiles == 1 or (tiles <= FUSED_BC_SHORT_MAX_TILES and
+                          2 * d_inner * d_state * 4 * d_inner * 2 <= FUSED_BC_SHORT_CACHED_BYTES)
 
 
 def fused_bc_eligible(x: torch.Tensor, B_weight: torch.Tensor, C_weight: torch.Tensor,

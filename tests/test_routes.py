@@ -309,3 +309,15 @@ def test_layernorm_backward_sizes():
     qn = importlib.import_module("mambaqc_amd.kernels.quaternion_norm")
     assert qn._sums_inside(16384, 8) and qn._sums_inside(300000, 192)
     assert not qn._sums_inside(16385, 191) and not qn._sums_inside(0, 64)
+
+
+def test_fused_prompt_sizes():
+    """Both sides of the lines that a prompt's fused form was measured at."""
+    wins = sf.fused_bc_short_wins
+    assert wins(1, 17, 1536, 64) and wins(1, 128, 1536, 64) and wins(2, 64, 1536, 64)
+    assert not wins(1, 16, 1536, 64) and not wins(2, 100, 1536, 64) and not wins(0, 100, 512, 16)
+    assert wins(4, 128, 512, 64) and not wins(5, 128, 512, 64) and not wins(4, 100, 1024, 64)
+    assert wins(12, 33, 512, 64) and not wins(16, 33, 512, 64) and not wins(16, 100, 1024, 16)
+    assert wins(1, 160, 1536, 64) and not wins(1, 159, 1536, 64) and wins(1, 129, 1536, 32)
+    assert not wins(1, 255, 1536, 48) and not wins(1, 255, 1024, 16) and not wins(2, 200, 512, 16)
+    assert wins(1, 129, 768, 48) and not wins(1, 129, 768, 40) and wins(1, 129, 512, 40)
