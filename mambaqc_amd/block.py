@@ -522,8 +522,11 @@ class QuaternionMamba2Block(nn.Module):
         x_in, z = xz.chunk(2, dim=-1)
         conv = self.conv1d.conv
         x_act = causal_conv1d_silu_step_(x_in, tail, conv.weight, conv.bias)
-        dt_raw, g_raw = _linear_pair(self.dt_proj, self.gate_proj, x_act)
-        Bq, Cq = _bc_pair(self.B_proj, self.C_proj, x_act, self.d_state)
+        four = self._small_projections(x_act)
+        if four is None:
+            four = (*_linear_pair(self.dt_proj, self.gate_proj, x_act),
+                    *_bc_pair(self.B_proj, self.C_proj, x_act, self.d_state))
+        dt_raw, g_raw, Bq, Cq = four
         y = _sf.ssm_forward_front_dl_state_(dt_raw, g_raw, x_act, Bq, Cq, self.Lambda_alpha,
                                             self.Lambda_imag, self.D, h, eps=1e-6)
         y_real = _out_proj(self.out_proj, self.norm(y))
@@ -615,18 +618,12 @@ class QuaternionMamba2Block(nn.Module):
             x.requires_grad or (h0 is not None and h0.requires_grad)
             or any(p.requires_grad for p in self.parameters()))
         width = self._bc_slice_width(x, recording)
-        dtp, gp, bp, cp = self.dt_proj, self.gate_proj, self.B_proj, self.C_proj
         Bq = Cq = None
-        if (not recording and not width and bp.bias is None and cp.bias is None
-                and _bare(nn.Linear, dtp, gp) and _bare(QuaternionLinear, bp, cp)
-                and f32_small_eligible(x, dtp.weight, dtp.bias, gp.weight, gp.bias,
-                                       bp.weight, None, cp.weight, None)):
-            # A small fp32 block: the four projections of x in one launch.
-            dt_raw, g_raw, Bq, Cq = f32_small_linears(x, dtp.weight, dtp.bias, gp.weight, gp.bias,
-                                                      bp.weight, None, cp.weight, None)
-            Bq, Cq = (m.view(b, t, D, self.d_state, 4) for m in (Bq, Cq))
+        four = None if recording or width else self._small_projections(x)
+        if four is not None:
+            dt_raw, g_raw, Bq, Cq = four
         else:
-            dt_raw, g_raw = _linear_pair(dtp, gp, x)
+            dt_raw, g_raw = _linear_pair(self.dt_proj, self.gate_proj, x)
         if not recording and self._use_fused_bc(x):
             delta, s = ssm_front(dt_raw, g_raw, x)
             # Under autocast the projections' operands in its dtype, as F.linear casts them.
@@ -650,6 +647,18 @@ class QuaternionMamba2Block(nn.Module):
         return ssm_forward_front_dl(dt_raw, g_raw, x, Bq, Cq, self.Lambda_alpha,
                                     self.Lambda_imag, self.D, eps=1e-6, h0=h0,
                                     return_state=return_state)
+
+    def _small_projections(self, x: torch.Tensor):
+        """dt, gate, B and C projections of x in one launch where they are small fp32 ones
+        (f32_small_eligible), else None."""
+        dtp, gp, bp, cp = self.dt_proj, self.gate_proj, self.B_proj, self.C_proj
+        args = (dtp.weight, dtp.bias, gp.weight, gp.bias, bp.weight, None, cp.weight, None)
+        if (bp.bias is not None or cp.bias is not None or not _bare(nn.Linear, dtp, gp)
+                or not _bare(QuaternionLinear, bp, cp) or not f32_small_eligible(x, *args)):
+            return None
+        dt_raw, g_raw, Bq, Cq = f32_small_linears(x, *args)
+        Bq, Cq = (m.view(*x.shape, self.d_state, 4) for m in (Bq, Cq))
+        return dt_raw, g_raw, Bq, Cq
 
     def _use_fused_bc(self, x: torch.Tensor) -> bool:
         """Whether this inference forward runs the B/C projections fused into the
