@@ -146,15 +146,17 @@ class _WideLinearFunction(torch.autograd.Function):
 # weight gradients 1990 / 1174 and 105 / 94. Below the lines: M 100 N 98304 K 384 86 / 120 (a short
 # side), 98304 x 384 over K 100 94 / 114 (short k: padding and output dominate), 1024 x 1024 x 1024
 # 22 / 35 (launches). An operand with its rows contiguous is read once more for the rows' maxima, so
-# the side that repays it is longer: with none (a forward) M 255 N 294912 K 1536 1622 / 1922, M 306
-# N 196608 K 768 737 / 666; with one (an input gradient) M 1602 N 320 K 51200 419 / 541, M 639 N 768
-# K 49152 432 / 456, M 1212 N 512 K 40960 481 / 352; with two (a weight gradient) M 49152 N 256 K 2203
-# 406 / 648, M 98304 N 384 K 5679 2878 / 3627, M 30720 N 384 K 5286 1132 / 970, M 98304 N 512 K 2427
-# 1717 / 1722, M 51200 N 640 K 523 270 / 236. An input gradient of few outputs leaves the library's
-# GEMM at 40-80 TFLOP/s and pays at any side from 200 on (M 973 N 256 K 24576 324 / 130, M 574 N 384
-# K 36864 327 / 199).
-F32_GEMM_MIN_SIDE = (256, 350, 500)  # M N / (M + N), by the operands with their rows contiguous
-F32_GEMM_FEW_OUTPUTS = 300_000       # up to this many, with one such operand at most:
+# the side that repays it depends on how many are: with none (a forward) M 255 N 294912 K 1536 1622 /
+# 1922, M 306 N 196608 K 768 737 / 666; with two (a weight gradient) M 49152 N 256 K 2203 406 / 648,
+# M 98304 N 384 K 5679 2878 / 3627, M 98304 N 512 K 2427 1717 / 1722, M 51200 N 640 K 523 270 / 236.
+# With one (an input gradient) the library's time is uneven (40 to 145 TFLOP/s): M 253 N 1536 K 294912
+# 2182 / 2386, M 313 N 1536 K 196608 1680 / 1725, M 1955 N 384 K 24576 638 / 249; of 55 shapes with
+# sides from 260 to 500 50 are faster here, half of them by 1.5 or more, and one slower by more
+# than 7 % (M 775 N 640 K 40960, 0.76 times as fast); with few outputs and k up to 65536 all measured
+# from 200 on are (M 973 N 256 K 24576 324 / 130), beyond that k not (M 384 N 640 K 163840 0.81).
+F32_GEMM_MIN_SIDE = (256, 260, 500)  # M N / (M + N), by the operands with their rows contiguous
+F32_GEMM_FEW_OUTPUTS = 300_000       # up to this many, with one such operand at most and k up to
+F32_GEMM_FEW_MAX_K = 1 << 16         # this:
 F32_GEMM_FEW_MIN_SIDE = 200
 F32_GEMM_MIN_K = 192
 F32_GEMM_MIN_FLOP = 6e9
@@ -164,7 +166,7 @@ def _f32_gemm_shape(M: int, N: int, K: int, by_rows: int = 0) -> bool:
     """Whether an fp32 product runs on mqc_gemm_f32, `by_rows` of its operands having their rows
     and not k contiguous."""
     side = F32_GEMM_MIN_SIDE[by_rows]
-    if by_rows < 2 and M * N <= F32_GEMM_FEW_OUTPUTS:
+    if by_rows < 2 and M * N <= F32_GEMM_FEW_OUTPUTS and K <= F32_GEMM_FEW_MAX_K:
         side = min(side, F32_GEMM_FEW_MIN_SIDE)
     return (K >= F32_GEMM_MIN_K and M * N >= side * (M + N)
             and 2.0 * M * N * K >= F32_GEMM_MIN_FLOP)

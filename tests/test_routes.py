@@ -275,7 +275,8 @@ def test_fp32_gemm_sizes():
     assert not takes(255, 294912, 1536) and not takes(100, 98304, 384)
     assert not takes(98304, 384, 100) and not takes(1024, 1024, 1024)
     assert takes(1024, 1024, 131072, 1) and takes(400, 512, 32768, 1) and takes(574, 384, 36864, 1)
-    assert not takes(1602, 320, 51200, 1) and not takes(639, 768, 49152, 1)
+    assert takes(1955, 384, 24576, 1) and not takes(253, 1536, 294912, 1)
+    assert not takes(384, 640, 163840, 1)
     assert takes(131072, 1024, 1024, 2) and takes(32768, 512, 400, 2)
     assert not takes(49152, 256, 2203, 2) and not takes(98304, 384, 5679, 2)
     x, w = torch.randn(6, 5), torch.randn(7, 5)
