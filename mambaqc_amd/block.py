@@ -229,9 +229,12 @@ def _bare(kind: type, *layers: nn.Module) -> bool:
     if (nat.compiling() or _module._global_forward_hooks or _module._global_forward_pre_hooks
             or _module._global_backward_hooks or _module._global_backward_pre_hooks):
         return False
-    return all(type(m) is kind and "forward" not in m.__dict__ and m._compiled_call_impl is None
-               and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                        or m._backward_pre_hooks) for m in layers)
+    for m in layers:
+        if (type(m) is not kind or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks or m._compiled_call_impl is not None
+                or "forward" in m.__dict__):
+            return False
+    return True
 
 
 def _linear(layer: nn.Linear, x: torch.Tensor) -> torch.Tensor:

@@ -16,6 +16,7 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 from torch.utils._device import DeviceContext
 
 from .. import _native as nat
@@ -243,24 +244,33 @@ class _F32MatmulT(torch.autograd.Function):
 
 
 def _function_modes() -> bool:
-    """Whether a TorchFunctionMode sees torch's calls, other than a default device's, which
-    leaves products alone."""
-    return torch._C._len_torch_function_stack() > 0 and not all(
-        type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+    """Whether a TorchFunctionMode other than a default device's, which leaves products alone,
+    sees torch's calls."""
+    return not all(type(m) is DeviceContext
+                   for m in torch.overrides._get_current_function_mode_stack())
+
+
+# (Looked up once: the check is on the host path of every small product.)
+_compiling, _tracing = torch.compiler.is_compiling, torch._C._is_tracing
+_len_functions, _len_dispatch = torch._C._len_torch_function_stack, torch._C._len_torch_dispatch_stack
+_interpreters, _has_storage = torch._C._functorch.peek_interpreter_stack, torch._C._has_storage
 
 
 def _plain_call(*tensors) -> bool:
     """Plain dense tensors called eagerly: no tensor subclass (fake tensors), no wrapper
     without storage (the batched gradients of autograd.grad, which show in no other way), no
     dispatch or function mode, tracing, functorch transform or forward-mode AD in progress, all
-    of which torch's own operators take part in and a direct launch does not."""
-    if torch.compiler.is_compiling() or _function_modes():
+    of which torch's own operators take part in and a direct launch does not. (None stands for
+    a bias that is not there.)"""
+    if (_compiling() or _len_dispatch() or _interpreters() is not None or _tracing()
+            or forward_ad._current_level >= 0 or _len_functions() and _function_modes()):
         return False
-    return (all(type(t) in (torch.Tensor, nn.Parameter) and t.layout == torch.strided
-                and torch._C._has_storage(t) and not t.is_neg() for t in tensors)
-            and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0)
+    for t in tensors:
+        if t is not None and not ((type(t) is nn.Parameter or type(t) is torch.Tensor)
+                                  and t.layout is torch.strided and _has_storage(t)
+                                  and not t.is_neg()):
+            return False
+    return True
 
 
 def _f32_linear_eligible(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -333,7 +343,7 @@ def f32_small_eligible(x: torch.Tensor, *params) -> bool:
         columns += w.shape[0]
     return (_f32_small_shape(rows, columns, K, len(params) // 2)
             and not torch.is_autocast_enabled(x.device.type)
-            and _plain_call(x, *(p for p in params if p is not None)))
+            and _plain_call(x, *params))
 
 
 def f32_small_linears(x: torch.Tensor, *params):
