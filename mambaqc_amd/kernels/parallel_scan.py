@@ -17,15 +17,20 @@ from .. import _native as nat
 # The time-chunked product (mqc_cumprod_scan_chunked) reads q twice, so it pays where the whole
 # walk is bound by its serial chain (us, whole / chunked): fp32 T 4096 1024 lanes 182 / 55, 4096
 # 188 / 146, but 8192 263 / 318; bf16 1024 433 / 44, 24576 (T 2000) 379 / 218, 16000 (T 256)
-# 30 / 25, 49152 (T 2000) 463 / 430. Short sequences leave little to save: bf16 T 128 12 / 17,
-# 192 16 / 17, 256 21 / 18, fp32 T 512 24 / 19.
+# 30 / 25, 49152 (T 2000) 463 / 430. Short sequences leave little to save, the more the fewer the
+# lanes (with the Cayley map that wrote q, bf16): T 128 1024 lanes 18.5 / 22.5, 2048 20 / 22.6, 6144
+# 27 / 22, 24576 36 / 31; T 160 256 lanes 23.3 / 22.8, 2048 26 / 23; T 234 16384 lanes 56 / 37.
 CHUNK_MAX_LANES = {4: 4096, 2: 24576}   # batch x lanes, by element size
-CHUNK_MIN_SEQ = {4: 512, 2: 256}
+CHUNK_MIN_SEQ = {4: 512, 2: 128}
+CHUNK_FEW_LANES = 4096                  # below this many:
+CHUNK_FEW_MIN_SEQ = {4: 512, 2: 160}
 
 
 def _chunk_len(B: int, T: int, lanes: int, el: int) -> int:
     """Steps per chunk, 0 for the whole walk."""
-    if B < 1 or lanes < 1 or B * lanes > CHUNK_MAX_LANES[el] or T < CHUNK_MIN_SEQ[el]:
+    if B < 1 or lanes < 1 or B * lanes > CHUNK_MAX_LANES[el]:
+        return 0
+    if T < (CHUNK_FEW_MIN_SEQ if B * lanes < CHUNK_FEW_LANES else CHUNK_MIN_SEQ)[el]:
         return 0
     L = nat.q_chunk_len(B, T, lanes, el)
     return L if L < T and B * -(-T // L) <= 65535 else 0

@@ -37,21 +37,22 @@ def _d_strides(D: torch.Tensor, dtype: torch.dtype):
 # The time-chunked q form (mqc_ssm_q_fwd_chunked) reads q and B twice, so it pays where the whole
 # walk is bound by its serial chain, 0.4 us a step (us, whole / chunked): fp32 T 4096 1024 lanes
 # 1649 / 80, 8192 1662 / 471, 24576 (T 2000) 821 / 662, but 49152 924 / 1367; bf16 8192 1614 / 268,
-# 49152 (T 2000) 799 / 782; T 150 3200 lanes 62 / 22. With most lanes short sequences are no longer
-# bound by the chain: fp32 24576 lanes T 64 32 / 33, 128 58 / 52; bf16 24576 T 64 31 / 28, but 49152
-# T 64 31 / 38, 256 106 / 111, 384 157 / 152.
-Q_CHUNK_MAX_BYTES = 96 << 10  # batch x lanes x element size
+# 49152 (T 2000) 799 / 782; T 150 3200 lanes 62 / 22. With most lanes the chain is hardly the
+# bound, least in short sequences (with the Cayley map that wrote q): fp32 24576 lanes T 64 37 / 42,
+# 128 72 / 68, 512 269 / 236; bf16 24576 T 64 35 / 34, 32768 T 100 52 / 54, 128 67 / 58, but 49152
+# T 128 71 / 82, 512 263 / 266.
+Q_CHUNK_MAX_BYTES = {4: 96 << 10, 2: 64 << 10}  # batch x lanes x element size, by element size
 Q_CHUNK_MIN_SEQ = 64
 Q_CHUNK_MANY_BYTES = 48 << 10  # above this:
-Q_CHUNK_MANY_MIN_SEQ = {4: 128, 2: 384}  # by element size
+Q_CHUNK_MANY_MIN_SEQ = 128
 
 
 def _q_chunk_len(batch: int, T: int, lanes: int, el: int) -> int:
     """Steps per chunk of the q form, 0 for the whole walk."""
     nbytes = batch * lanes * el
-    if batch < 1 or lanes < 1 or nbytes > Q_CHUNK_MAX_BYTES or el not in Q_CHUNK_MANY_MIN_SEQ:
+    if batch < 1 or lanes < 1 or nbytes > Q_CHUNK_MAX_BYTES.get(el, 0):
         return 0
-    if T < (Q_CHUNK_MANY_MIN_SEQ[el] if nbytes > Q_CHUNK_MANY_BYTES else Q_CHUNK_MIN_SEQ):
+    if T < (Q_CHUNK_MANY_MIN_SEQ if nbytes > Q_CHUNK_MANY_BYTES else Q_CHUNK_MIN_SEQ):
         return 0
     L = nat.q_chunk_len(batch, T, lanes, el)
     return L if L < T and batch * -(-T // L) <= 65535 else 0

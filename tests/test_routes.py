@@ -297,13 +297,14 @@ def test_small_fp32_sizes():
 
 def test_chunked_scan_sizes():
     """Both sides of the lines on lanes and steps, and no chunks for another element size."""
-    for el, short, long in ((4, 511, 512), (2, 255, 256)):
-        assert not ps._chunk_len(1, short, 1024, el) and ps._chunk_len(1, long, 1024, el)
+    for el, lanes, short, long in ((4, 1024, 511, 512), (2, 1024, 159, 160), (2, 4096, 127, 128)):
+        assert not ps._chunk_len(1, short, lanes, el) and ps._chunk_len(1, long, lanes, el)
     assert ps._chunk_len(1, 4096, 4096, 4) and not ps._chunk_len(1, 4096, 4097, 4)
     assert sf._q_chunk_len(1, 64, 12288, 4) and not sf._q_chunk_len(1, 64, 24576, 4)
     assert sf._q_chunk_len(1, 128, 24576, 4) and not sf._q_chunk_len(1, 4096, 24577, 4)
-    assert sf._q_chunk_len(1, 64, 24576, 2) and not sf._q_chunk_len(2, 383, 24576, 2)
-    assert sf._q_chunk_len(2, 384, 24576, 2) and not sf._q_chunk_len(1, 600, 64, 8)
+    assert sf._q_chunk_len(1, 64, 24576, 2) and not sf._q_chunk_len(2, 127, 16384, 2)
+    assert sf._q_chunk_len(2, 128, 16384, 2) and not sf._q_chunk_len(2, 4096, 24576, 2)
+    assert not sf._q_chunk_len(1, 600, 64, 8)
 
 
 def test_layernorm_backward_sizes():
