@@ -582,6 +582,14 @@ def fused_bc_short_wins(batch: int, seq_len: int, d_inner: int, d_state: int) ->
                           2 * d_inner * d_state * 4 * d_inner * 2 <= FUSED_BC_SHORT_CACHED_BYTES)
 
 
+def fused_bc_short_rows(batch: int, seq_len: int, d_inner: int, d_state: int) -> int:
+    """Batch rows that one launch of the short form takes: as many as its 32-bit unit index counts
+    and as have their partial sums (8 times y at 64 states) within FUSED_BC_SPLIT_WS_MAX."""
+    row = nat.load().mqc_ssm_fused_bc_short_workspace_bytes(1, seq_len, d_inner, d_state)
+    rows = min(batch, 0x7fffffff // (d_inner * 64))
+    return max(1, min(rows, FUSED_BC_SPLIT_WS_MAX // row)) if row else max(1, rows)
+
+
 def fused_bc_eligible(x: torch.Tensor, B_weight: torch.Tensor, C_weight: torch.Tensor,
                       d_state: int, dtype: torch.dtype | None = None) -> bool:
     """Whether ssm_forward_fused_bc takes these operands: x [batch, T, d_inner] with
@@ -619,7 +627,8 @@ def ssm_forward_fused_bc(x: torch.Tensor, B_weight: torch.Tensor, C_weight: torc
     split: run each half of the states (32) in a workgroup of its own, with a
     workspace for the halves' partial sums and a second launch adding them (the
     same y bit for bit); None splits batches of at most FUSED_BC_SPLIT_MAX_BATCH, and
-    runs sequences of at most FUSED_BC_SHORT_MAX_SEQ tokens in the short form.
+    runs sequences of at most FUSED_BC_SHORT_MAX_SEQ tokens in the short form (in
+    launches of fused_bc_short_rows batch rows).
     """
     batch, T, d_inner = x.shape
     d_state = lambda_alpha.shape[-1] if lambda_alpha.dim() == 2 else 0
@@ -652,13 +661,18 @@ def ssm_forward_fused_bc(x: torch.Tensor, B_weight: torch.Tensor, C_weight: torc
     h_last = (torch.empty(batch, d_inner, d_state, 4, device=x.device, dtype=torch.float32)
               if return_state else None)
     lib = nat.load()
-    if split is None and 0 < T <= FUSED_BC_SHORT_MAX_SEQ:
-        ws_bytes = lib.mqc_ssm_fused_bc_short_workspace_bytes(batch, T, d_inner, d_state)
+    if split is None and 0 < T <= FUSED_BC_SHORT_MAX_SEQ and batch and d_inner:
+        rows = fused_bc_short_rows(batch, T, d_inner, d_state)
+        ws_bytes = lib.mqc_ssm_fused_bc_short_workspace_bytes(rows, T, d_inner, d_state)
         ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8) if ws_bytes else None
-        nat.call("mqc_ssm_fused_bc_short_fwd", xc, xc.data_ptr(), wb.data_ptr(), wc.data_ptr(),
-                 dl.data_ptr(), sv.data_ptr(), la.data_ptr(), li.data_ptr(), Dv.data_ptr(),
-                 nat.ptr(h0c), y.data_ptr(), nat.ptr(h_last), batch, T, d_inner, d_state,
-                 float(eps), code, nat.ptr(ws), ws_bytes, nat.stream_of(xc))
+        stream = nat.stream_of(xc)
+        for b0 in range(0, batch, rows):  # (in the stream's order, so one workspace serves all)
+            b1 = min(batch, b0 + rows)
+            nat.call("mqc_ssm_fused_bc_short_fwd", xc, xc[b0:b1].data_ptr(), wb.data_ptr(),
+                     wc.data_ptr(), dl[b0:b1].data_ptr(), sv[b0:b1].data_ptr(), la.data_ptr(),
+                     li.data_ptr(), Dv.data_ptr(), None if h0c is None else h0c[b0:b1].data_ptr(),
+                     y[b0:b1].data_ptr(), None if h_last is None else h_last[b0:b1].data_ptr(),
+                     b1 - b0, T, d_inner, d_state, float(eps), code, nat.ptr(ws), ws_bytes, stream)
         return (y, h_last) if return_state else y
     if split is None:
         split = batch <= FUSED_BC_SPLIT_MAX_BATCH

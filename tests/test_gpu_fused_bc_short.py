@@ -72,6 +72,22 @@ def test_short_keeps_sequences_apart():
     assert y[1].isnan().all()
 
 
+@pytest.mark.parametrize("with_h0", [False, True])
+def test_short_in_several_launches(with_h0, monkeypatch):
+    """A batch beyond one launch's rows: the same numbers from launches of 4, 4 and 1."""
+    from mambaqc_amd.kernels import ssm_fused as sf
+    b, T, d, k = 9, 21, 64, 48
+    x, wb, wc, delta, s, la, li, D, h0 = _inputs(b, T, d, k, seed=6)
+    h0 = h0 if with_h0 else None
+    with torch.no_grad():
+        want, hw = K.ssm_forward_fused_bc(x, wb, wc, delta, s, la, li, D, h0=h0, return_state=True)
+        space = nat.load().mqc_ssm_fused_bc_short_workspace_bytes
+        monkeypatch.setattr(sf, "FUSED_BC_SPLIT_WS_MAX", 4 * space(1, T, d, k))
+        assert sf.fused_bc_short_rows(b, T, d, k) == 4
+        y, h = K.ssm_forward_fused_bc(x, wb, wc, delta, s, la, li, D, h0=h0, return_state=True)
+    assert torch.equal(y, want) and torch.equal(h, hw)
+
+
 def test_block_takes_it_for_prompts():
     torch.manual_seed(0)
     blk = QuaternionMamba2Block(64, d_state=16).to(DEV, BF)

@@ -323,3 +323,16 @@ def test_fused_prompt_sizes():
     assert wins(1, 160, 1536, 64) and not wins(1, 159, 1536, 64) and wins(1, 129, 1536, 32)
     assert not wins(1, 255, 1536, 48) and not wins(1, 255, 1024, 16) and not wins(2, 200, 512, 16)
     assert wins(1, 129, 768, 48) and not wins(1, 129, 768, 40) and wins(1, 129, 512, 40)
+
+
+def test_short_form_of_large_batches():
+    """Batches whose units pass the short form's 32-bit index (its entry point refuses them), or
+    whose partial sums would pass the fused scans' workspace bound, go in launches of fewer rows."""
+    rows = sf.fused_bc_short_rows
+    assert rows(1, 100, 1536, 64) == 1 and rows(64, 128, 1536, 64) == 64
+    assert rows(4096, 128, 1536, 64) == sf.FUSED_BC_SPLIT_WS_MAX // (4 * 128 * 1536 * 16)
+    assert rows(21845, 16, 1536, 16) == 21845 and rows(21846, 16, 1536, 16) == 21845
+    args = [ctypes.c_void_p(4096)] * 11  # (never read: a size or the workspace is refused first)
+    for batch, status in ((21846, -5), (21845, -1)):
+        assert nat.load().mqc_ssm_fused_bc_short_fwd(*args, batch, 16, 1536, 32, 1e-6, nat.BF16,
+                                                     None, 0, None) == status
