@@ -297,12 +297,14 @@ F32_SMALL_MAX_K = (512, 1024)        # for one product in the launch, for severa
 F32_SMALL_FEW_ROWS = 32              # below this many rows:
 F32_SMALL_FEW_ROWS_MAX_K = (64, 256)
 F32_SMALL_MAX_WEIGHT_BYTES = 16 << 20  # per product
+F32_SMALL_MAX_SIDE = 1 << 24  # the kernel's own limit on rows and columns
 
 
 def _f32_small_shape(M: int, N: int, K: int, count: int = 1) -> bool:
     """Whether `count` products of M rows and N columns together run on mqc_gemm_f32_small."""
     max_k = (F32_SMALL_MAX_K if M >= F32_SMALL_FEW_ROWS else F32_SMALL_FEW_ROWS_MAX_K)[count > 1]
-    return (M > 0 and N > 0 and 0 < K <= max_k and 2.0 * M * N * K <= F32_SMALL_MAX_FLOP
+    return (0 < M <= F32_SMALL_MAX_SIDE and 0 < N <= F32_SMALL_MAX_SIDE and 0 < K <= max_k
+            and 2.0 * M * N * K <= F32_SMALL_MAX_FLOP
             and 4 * N * K <= count * F32_SMALL_MAX_WEIGHT_BYTES)
 
 

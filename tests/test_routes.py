@@ -293,6 +293,10 @@ def test_small_fp32_sizes():
         assert takes(rows, 256, 64) and takes(rows, 2 * 128 + 2 * 8192, 128, 4)
         assert not takes(rows, 1024, 256) and not takes(rows, 3072, 1536, 2)
         assert not takes(rows, 2048, 2048) and not takes(rows, 262144, 1024, 2)
+    # Very long and very thin: the kernel's entry point refuses more rows than this.
+    product = (ctypes.c_int64 * 11)(4096, 2, 1, 4096, 2, 1, 0, 4096, (1 << 24) + 1, 2, 2)
+    assert nat.load().mqc_gemm_f32_small(product, 1, None) == -5
+    assert takes(1 << 24, 2, 2) and not takes((1 << 24) + 1, 2, 2) and not takes(2, (1 << 24) + 1, 2)
 
 
 def test_chunked_scan_sizes():
