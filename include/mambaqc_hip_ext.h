@@ -33,8 +33,8 @@ int mqc_gemm_f32(const float* X, int64_t x_row, int64_t x_col, const float* W, i
  * bias (or 0), Y, M, N, K (pointers as integers; one of xm, xk and one of wn, wk is 1). */
 int mqc_gemm_f32_small(const int64_t* products, int64_t count, void* stream);
 
-/* mqc_qln_bwd with its parameter sums: dq, and dgamma [d] and dbeta [d, 4] in fp32. rows and d at least 1, d at most 4096; workspace of
- * mqc_qln_bwd_sums_workspace_bytes(rows, d). */
+/* mqc_qln_bwd with its parameter sums: dq, and dgamma [d] and dbeta [d, 4] in fp32. rows and d at
+ * least 1, d at most 4096; workspace of mqc_qln_bwd_sums_workspace_bytes(rows, d). */
 int64_t mqc_qln_bwd_sums_workspace_bytes(int64_t rows, int64_t d);
 int mqc_qln_bwd_sums(const void* q, const void* dout, const float* gamma, const float* mean,
                      const float* rstd, void* dq, float* dgamma, float* dbeta, int64_t rows,
@@ -56,11 +56,11 @@ int64_t mqc_q_chunked_workspace_bytes(int64_t batch, int64_t seq_len, int64_t la
 int mqc_cumprod_scan_chunked(const void* q, void* out, int64_t batch, int64_t seq_len,
                              int64_t lanes, int64_t chunk_len, int dtype, void* workspace,
                              int64_t workspace_bytes, void* stream);
-int mqc_ssm_q_fwd_chunked(const void* q, const void* B, const void* Sq, const void* C, const void* D,
-                          int64_t d_stride_b, int64_t d_stride_t, int64_t d_stride_d, void* y,
-                          int64_t batch, int64_t seq_len, int64_t d_model, int64_t d_state,
-                          int64_t chunk_len, int dtype, void* workspace, int64_t workspace_bytes,
-                          void* stream);
+int mqc_ssm_q_fwd_chunked(const void* q, const void* B, const void* Sq, const void* C,
+                          const void* D, int64_t d_stride_b, int64_t d_stride_t,
+                          int64_t d_stride_d, void* y, int64_t batch, int64_t seq_len,
+                          int64_t d_model, int64_t d_state, int64_t chunk_len, int dtype,
+                          void* workspace, int64_t workspace_bytes, void* stream);
 
 /* mqc_ssm_fused_bc_fwd for short sequences, seq_len from 1 to 128 (MQC_E_LIMIT above): same
  * operands, dtypes, shapes and refusals, in tiles of 64 or 128 tokens that hold whole

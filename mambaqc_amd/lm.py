@@ -174,7 +174,8 @@ class QuaternionMamba2(nn.Module):
 class DecodeGraph:
     """One recurrent decode step of a QuaternionMamba2 (a token per sequence
     through every block) captured as a HIP graph, for serving loops where the
-    step's ~12 kernels per layer would otherwise each be launched from Python.
+    step's kernels (four per layer at decode batches, about twelve where the fused
+    step does not apply) would otherwise each be launched from Python.
 
     The graph reads its tokens and the per-layer states (conv tails, fp32 SSM
     states) from static buffers and its kernels update those states in place
