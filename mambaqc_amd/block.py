@@ -242,7 +242,8 @@ def _linear(layer: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     small fp32 ones."""
     if skinny_eligible(x, layer.weight, layer.bias):
         return skinny_linear(x, layer.weight, layer.bias)
-    if _bare(nn.Linear, layer) and f32_small_eligible(x, layer.weight, layer.bias):
+    if (x.dtype == torch.float32 and _bare(nn.Linear, layer)
+            and f32_small_eligible(x, layer.weight, layer.bias)):
         return f32_small_linears(x, layer.weight, layer.bias)[0]
     return layer(x)
 
@@ -251,7 +252,8 @@ def _linear_pair(a: nn.Linear, b: nn.Linear, x: torch.Tensor):
     """(a(x), b(x)), in one skinny launch for decode-sized inputs."""
     if skinny_eligible(x, a.weight, a.bias, b.weight, b.bias):
         return skinny_linear(x, a.weight, a.bias, b.weight, b.bias)
-    if _bare(nn.Linear, a, b) and f32_small_eligible(x, a.weight, a.bias, b.weight, b.bias):
+    if (x.dtype == torch.float32 and _bare(nn.Linear, a, b)
+            and f32_small_eligible(x, a.weight, a.bias, b.weight, b.bias)):
         return f32_small_linears(x, a.weight, a.bias, b.weight, b.bias)
     return a(x), b(x)
 
@@ -654,6 +656,8 @@ class QuaternionMamba2Block(nn.Module):
     def _small_projections(self, x: torch.Tensor):
         """dt, gate, B and C projections of x in one launch where they are small fp32 ones
         (f32_small_eligible), else None."""
+        if x.dtype != torch.float32:  # (before reading eight parameters from their modules)
+            return None
         dtp, gp, bp, cp = self.dt_proj, self.gate_proj, self.B_proj, self.C_proj
         args = (dtp.weight, dtp.bias, gp.weight, gp.bias, bp.weight, None, cp.weight, None)
         if (bp.bias is not None or cp.bias is not None or not _bare(nn.Linear, dtp, gp)
